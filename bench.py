@@ -79,7 +79,7 @@ def measured_traffic(config, stage, block):
     committed rocprofv3 FETCH_SIZE / WRITE_SIZE passes (profiles/pmc_traffic_<workload>.json,
     copy-calibrated); None where no measurement of this workload and block size is committed."""
     kern = {"shift": f"k_fluid_shift<sphnj::M32, {block}>",
-            "fluid": f"k_fluid_pair_update<sphnj::M32, false, {block}>", "cells": None}[stage]
+            "fluid": f"k_fluid_pair_update<sphnj::M32, false, {block}", "cells": None}[stage]
     f = ROOT / "profiles" / {"two_phase": "pmc_traffic_two_phase_3M.json"}.get(config, "-")
     if kern is None or not f.exists():
         return None
@@ -94,7 +94,7 @@ def measured_issue(config, stage, block):
     the committed rocprofv3 SQ_INSTS_VALU / GRBM_GUI_ACTIVE pass (profiles/pmc_valu_<workload>.json;
     a CU issues at most about one wave64 VALU instruction per cycle); None where not measured."""
     kern = {"shift": f"k_fluid_shift<sphnj::M32, {block}>",
-            "fluid": f"k_fluid_pair_update<sphnj::M32, false, {block}>", "cells": None}[stage]
+            "fluid": f"k_fluid_pair_update<sphnj::M32, false, {block}", "cells": None}[stage]
     f = ROOT / "profiles" / {"two_phase": "pmc_valu_two_phase_3M.json"}.get(config, "-")
     if kern is None or not f.exists():
         return None

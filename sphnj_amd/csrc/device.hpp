@@ -25,8 +25,8 @@ struct M32 {
 template <class R>
 struct CaseDev {
   // kernel (Kernel::initiate, src/kernel.cpp:25-41)
-  R rc2, hinv2, kdc, k2c, eR, h, eps_h2;  // eps_h2 = 0.01 h^2
-  R nhl2;  // -hinv2 * log2(e): exp(-r^2/h^2) = 2^(r^2 nhl2)
+  R rc2, kdc, k2c, eR, h, eps_h2;  // eps_h2 = 0.01 h^2
+  R nhl2;  // -log2(e) / h^2: exp(-r^2/h^2) = 2^(r^2 nhl2)
   // scaled units of the M32 shift loop: x' = x sqrt(hinv2 log2 e), so exp(-r^2/h^2) = 2^-r'^2
   float gscale, rc2s, kdc_s;  // scale, rc^2 scaled, kd c32 / scale
   R quarter_rc2;
@@ -225,23 +225,53 @@ __device__ __forceinline__ int axis_sub(double x, double x0, double inv, int n, 
   return 2 * c + h;
 }
 
+// exp(-r^2/h^2) = 2^(r2 nhl2), nhl2 = -log2(e)/h^2.
+//
+// FP64: with n the integer nearest to y = r2 nhl2 and f = y - n in [-1/2, 1/2], formed by one
+// fused multiply-add from the exact product, 2^f = 1 + f q(f) and n goes into the exponent.  q
+// (degree 10) interpolates (2^f - 1)/f at the Chebyshev nodes of the interval; with the
+// coefficients rounded to double 2^f is off by at most 2.0e-17 before the rounding of its own
+// arithmetic.  15 instructions, 14 of them FP64 (the library's exp takes about 40 with its range
+// handling).  n below -1000 gives 2^-1000 instead of leaving the exponent's range; an r2 far past
+// the cut-off (padding) gives a number that the caller's cut-off test discards.
+// FP32: v_exp_f32 computes 2^x.
 template <class R>
-__device__ __forceinline__ R kexp(R x);
+__device__ __forceinline__ R kgauss(R r2, R nhl2);
 template <>
-__device__ __forceinline__ double kexp<double>(double x) {
-  return exp(x);
+__device__ __forceinline__ double kgauss<double>(double r2, double nhl2) {
+  constexpr double kRound = 6755399441055744.0;  // 1.5 * 2^52: the sum's low word is n
+  const double t = fma(r2, nhl2, kRound);
+  const double f = fma(r2, nhl2, -(t - kRound));
+  double q = 0x1.e9d3fe3ccce58p-32;
+  q = fma(q, f, 0x1.e6063f762c3fep-28);
+  q = fma(q, f, 0x1.b524fae625c5ep-24);
+  q = fma(q, f, 0x1.62bfd477712afp-20);
+  q = fma(q, f, 0x1.ffcbfc670dcddp-17);
+  q = fma(q, f, 0x1.430913096fdaap-13);
+  q = fma(q, f, 0x1.5d87fe78a5276p-10);
+  q = fma(q, f, 0x1.3b2ab6fba1ddap-7);
+  q = fma(q, f, 0x1.c6b08d704a0c2p-5);
+  q = fma(q, f, 0x1.ebfbdff82c598p-3);
+  q = fma(q, f, 0x1.62e42fefa39efp-1);
+  q = fma(q, f, 1.0);
+  const int n = max(__double2loint(t), -1000);
+  return __hiloint2double(__double2hiint(q) + (n << 20), __double2loint(q));
 }
 template <>
-__device__ __forceinline__ float kexp<float>(float x) {
-  // v_exp_f32 computes 2^x; arguments here lie in [-R^2 log2 e, 0]
-  return __builtin_amdgcn_exp2f(x * 1.4426950408889634f);
+__device__ __forceinline__ float kgauss<float>(float r2, float nhl2) {
+  return __builtin_amdgcn_exp2f(r2 * nhl2);
 }
 
+// 1/sqrt(x) and 1/x.  FP64: the hardware's estimate y (relative error e/2 or e, about 2^-23) and
+// one third-order step, whose own error is below 2^-63: 6 and 4 instructions, where a correctly
+// rounded square root and division take about 20 and 10.
 template <class R>
 __device__ __forceinline__ R krsqrt(R x);
 template <>
 __device__ __forceinline__ double krsqrt<double>(double x) {
-  return 1.0 / sqrt(x);
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 template <>
 __device__ __forceinline__ float krsqrt<float>(float x) {
@@ -252,11 +282,26 @@ template <class R>
 __device__ __forceinline__ R krcp(R x);
 template <>
 __device__ __forceinline__ double krcp<double>(double x) {
-  return 1.0 / x;
+  const double y = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, y, 1.0);
+  return fma(y, fma(e, e, e), y);
 }
 template <>
 __device__ __forceinline__ float krcp<float>(float x) {
   return __builtin_amdgcn_rcpf(x);
+}
+
+// a / b.  FP64: the product with 1/b and its residual's correction.
+template <class R>
+__device__ __forceinline__ R kdiv(R a, R b);
+template <>
+__device__ __forceinline__ double kdiv<double>(double a, double b) {
+  const double y = krcp<double>(b), q = a * y;
+  return fma(fma(-b, q, a), y, q);
+}
+template <>
+__device__ __forceinline__ float kdiv<float>(float a, float b) {
+  return a / b;
 }
 
 __device__ __forceinline__ unsigned long long wave_max_u64(unsigned long long v) {

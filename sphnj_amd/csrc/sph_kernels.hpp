@@ -97,6 +97,9 @@ __device__ __forceinline__ bool cell_run(const Dev<Pol> &d, const CP &cp, int cx
   return true;
 }
 
+__device__ __forceinline__ float kfma(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
+__device__ __forceinline__ double kfma(double a, double b, double c) { return __builtin_fma(a, b, c); }
+
 // Sum over the aligned groups of W lanes (W a power of two dividing 64).
 template <int W, class T>
 __device__ __forceinline__ T lanes_sum(T v) {
@@ -525,7 +528,7 @@ __global__ void __launch_bounds__(256) k_wall_normal(Dev<Pol> d) {
         const R dx = d.w_vx[s] - bx, dy = d.w_vy[s] - by;
         const R r2 = dx * dx + dy * dy;
         if (r2 < cp.rc2) {
-          const R w = kexp<R>(-(r2 * cp.hinv2)) * cp.kdc;
+          const R w = kgauss<R>(r2, cp.nhl2) * cp.kdc;
           nx -= dx * w;
           ny -= dy * w;
         }
@@ -581,7 +584,7 @@ __device__ __forceinline__ void wall_update_block(const Dev<Pol> &d, int bid) {
           const R dx = F.vx[s] - bx, dy = F.vy[s] - by;
           const R r2 = dx * dx + dy * dy;
           if (!(r2 < cp.rc2)) continue;
-          const R w = (kexp<R>(-(r2 * cp.hinv2)) - cp.eR) * cp.k2c;
+          const R w = (kgauss<R>(r2, cp.nhl2) - cp.eR) * cp.k2c;
           S[j] += w;
           U[j] += F.vu[s] * w;
           V[j] += F.vv[s] * w;
@@ -1444,83 +1447,116 @@ __device__ __forceinline__ void for_range_4_2_1(int lo, int hi, F &&f) {
 // Per-case constants a neighbour loop needs, held in registers.
 template <class R>
 struct LoopConsts {
-  R rc2, nhl2, hinv2, kdc;
+  R rc2, nhl2, kdc;
   template <class CP>
-  __device__ __forceinline__ explicit LoopConsts(const CP &cp)
-      : rc2(cp.rc2), nhl2(cp.nhl2), hinv2(cp.hinv2), kdc(cp.kdc) {}
-  // Gradient weight w'(r^2) = exp(-r^2/h^2) kd c32 inside the cut-off, exactly 0 outside, so a
-  // candidate outside the cut-off adds exact zeros and the loop needs no branch.
-  __device__ __forceinline__ R w(R r2) const {
-    R e;
-    if constexpr (sizeof(R) == 4)
-      e = __builtin_amdgcn_exp2f(r2 * nhl2);
-    else
-      e = exp(-(r2 * hinv2));
-    return r2 < rc2 ? e * kdc : R(0);
+  __device__ __forceinline__ explicit LoopConsts(const CP &cp) : rc2(cp.rc2), nhl2(cp.nhl2), kdc(cp.kdc) {}
+  // exp(-r^2/h^2) inside the cut-off, exactly 0 outside, so a candidate outside the cut-off adds
+  // exact zeros and the loop needs no branch
+  __device__ __forceinline__ R gauss(R r2) const {
+    const R e = kgauss<R>(r2, nhl2);
+    return r2 < rc2 ? e : R(0);
   }
-  // w'(r^2) of a candidate known to lie inside the cut-off
-  __device__ __forceinline__ R w_in(R r2) const {
-    if constexpr (sizeof(R) == 4)
-      return __builtin_amdgcn_exp2f(r2 * nhl2) * kdc;
-    else
-      return exp(-(r2 * hinv2)) * kdc;
-  }
+  // the same of a candidate known to lie inside the cut-off
+  __device__ __forceinline__ R gauss_in(R r2) const { return kgauss<R>(r2, nhl2); }
+  // gradient weight w'(r^2) = exp(-r^2/h^2) kd c32, 0 outside the cut-off
+  __device__ __forceinline__ R w(R r2) const { return gauss(r2) * kdc; }
 };
 
 // ======================================================================================
 // FLUID: Riemann pair loop fused with the explicit update
 // ======================================================================================
 
+// Sums over a lane's neighbours, with the factors that a lane's terms share left out (pair_finish
+// multiplies them in once): ax, ay without -2 kd c32 / rho_i, drho without 2 kd c32, L without
+// -kd c32 and col without kd c32.
 template <class R>
 struct PairSums {
   R ax = 0, ay = 0, drho = 0, L00 = 0, L01 = 0, L10 = 0, L11 = 0, col = 0;
-  R fsr = R(1e30);  // smallest r^2 of a FREE_SURFACE neighbour inside the cut-off (liquid lanes)
+  R fsr = R(1e30);  // smallest r^2 of a FREE_SURFACE neighbour inside the cut-off
 };
-
-// Riemann terms of fluidFluidCalculate / fluidSolidCalculate / fluidVirtCalculate
-// (src/fluid.cu:25-191), with the algebra rearranged around q = (u_i - u_j).dx:
-//   du = q / r,  (u_i - v*).dx = rho_j q / (rho_i + rho_j) - (p_i - p_j) r / ((rho_i + rho_j) c).
-template <class R, bool VISCID>
-__device__ __forceinline__ void riemann_pair(R dx, R dy, R r2, R w, R ui, R vi, R uj, R vj, R rhoi, R rhoi_inv,
-                                             R rhoj, R pi, R pj, R cs, R csinv, R mu8, R eps_h2, PairSums<R> &A) {
-  const R inv_r = r2 > R(0) ? krsqrt<R>(r2) : R(0);
-  const R rn = r2 * inv_r;  // |dx|
-  const R du_ = ui - uj, dv_ = vi - vj;
-  const R q = du_ * dx + dv_ * dy;
-  // the density weights rho_i / (rho_i + rho_j) and rho_j / (rho_i + rho_j); the factors that
-  // depend on particle i alone (-2 / rho_i, 2 rho_i, p_i / c) are formed once per lane
-  const R isum = krcp<R>(rhoi + rhoj);
-  const R ai = rhoi * isum, aj = rhoj * isum;
-  R ps = ai * pj + aj * pi;
-  const R du = q * inv_r;
-  if (du >= R(0)) ps += (rhoi * aj) * du * fmin(R(3) * du, cs);
-  const R t = (pi * csinv - pj * csinv) * isum;
-  const R s = ps * ((R(-2) * rhoi_inv) * w);
-  A.ax += s * dx;
-  A.ay += s * dy;
-  A.drho += ((R(2) * rhoi) * w) * (aj * q - t * rn);
-  const R wdx = w * dx, wdy = w * dy;
-  A.L00 -= du_ * wdx;
-  A.L01 -= du_ * wdy;
-  A.L10 -= dv_ * wdx;
-  A.L11 -= dv_ * wdy;
-  if constexpr (VISCID) {
-    const R vis = -q / (r2 + eps_h2);
-    const R tv = mu8 * vis * rhoi_inv * w;
-    A.ax += tv * dx;
-    A.ay += tv * dy;
-  }
+template <class R>
+__device__ __forceinline__ void pair_finish(PairSums<R> &A, R rhoi, R kdc) {
+#pragma clang fp contract(off)
+  const R s = (R(-2) * kdc) * krcp<R>(rhoi);
+  A.ax *= s;
+  A.ay *= s;
+  A.drho *= R(2) * kdc;
+  A.L00 *= -kdc;
+  A.L01 *= -kdc;
+  A.L10 *= -kdc;
+  A.L11 *= -kdc;
+  A.col *= kdc;
 }
 
-// LDS capacity (particles) of a tile of BLOCK slots: the planner's budget.  The M32 pair kernel
-// (25 B of LDS per candidate) stages five eighths of it: a dense 256-lane tile over both
-// sub-columns of a cell column stages about 870 candidates, and at 37 KB per block with its
-// registers held to 104 (no spills) four blocks share a CU (16 waves instead of 12: 6%
-// faster).  FP64 candidates take 49 B, so P64 keeps the full budget.
-template <class Pol, int BLOCK>
+template <class R>
+__device__ __forceinline__ R norm2(R dx, R dy) {
+#pragma clang fp contract(off)
+  return kfma(dx, dx, dy * dy);
+}
+
+// Riemann terms of fluidFluidCalculate / fluidSolidCalculate / fluidVirtCalculate
+// (src/fluid.cu:25-191), with the algebra rearranged around q = (u_i - u_j).dx, d = p_j - p_i and
+// a = rho_i / (rho_i + rho_j):
+//   du = q / r,  p* = p_i + a d + a rho_j max(du, 0) min(3 du, c_i),
+//   (u_i - v*).dx = (rho_j q + d r / c_i) / (rho_i + rho_j),
+// and w = exp(-r^2/h^2) (0 outside the cut-off), so that every factor a lane's terms share comes
+// in once, in pair_finish.  d is formed first: equal pressures give exact zeros.  r^2 is kept off 0
+// for the root only; at r = 0 every term is 0 through dx, dy and q.  These terms are more than half
+// of the pair kernel's vector instructions, which is what bounds it: 121 per two candidates with
+// their fetch, against 136 with the density weights of both sides, the lane's factors in every
+// term and a test for r = 0.  464 -> 437 us a launch on the 3.0 M two-phase dam break (M32),
+// 922 -> 866 us (P64).
+// Every multiply-add is written out and contraction is off: what a lane sums must not depend on
+// how the compiler happens to fuse an instance of the kernel (block sizes, staged or global
+// candidates), and does not.
+template <class R, bool VISCID>
+__device__ __forceinline__ void riemann_pair(R dx, R dy, R r2, R w, R ui, R vi, R uj, R vj, R rhoi, R rhoj, R pi, R pj,
+                                             R cs, R csinv, R hmu, R eps_h2, PairSums<R> &A) {
+#pragma clang fp contract(off)
+  const R inv_r = krsqrt<R>(fmax(r2, sizeof(R) == 4 ? R(1e-36) : R(1e-290)));
+  const R rn = r2 * inv_r;  // |dx|
+  const R du_ = ui - uj, dv_ = vi - vj;
+  const R q = kfma(du_, dx, dv_ * dy);
+  const R d = pj - pi;
+  const R a = rhoi * krcp<R>(rhoi + rhoj);
+  const R du = fmax(q * inv_r, R(0));
+  R ps = kfma(a, d, pi);
+  ps = kfma((a * rhoj) * du, fmin(R(3) * du, cs), ps);
+  if constexpr (VISCID) ps = kfma(hmu, kdiv<R>(q, r2 + eps_h2), ps);  // hmu = 4 mu
+  A.drho = kfma(w * a, kfma(d, csinv * rn, rhoj * q), A.drho);
+  const R wdx = w * dx, wdy = w * dy;
+  A.ax = kfma(ps, wdx, A.ax);
+  A.ay = kfma(ps, wdy, A.ay);
+  A.L00 = kfma(du_, wdx, A.L00);
+  A.L01 = kfma(du_, wdy, A.L01);
+  A.L10 = kfma(dv_, wdx, A.L10);
+  A.L11 = kfma(dv_, wdy, A.L11);
+}
+
+// LDS capacity (particles) of a tile of BLOCK slots.  The planner's budget (plan_cap) holds the
+// tiles of any sensible spacing, but a dense 256-lane tile over both sub-columns of a cell column
+// stages about 870 candidates, and the LDS a block takes is what bounds the waves a CU holds:
+//  * M32 (25 B a candidate) stages five eighths of the budget: 37 KB a block and registers held to
+//    104 put four 256-lane blocks on a CU (16 waves instead of 12: 6% faster).
+//  * P64 (49 B) stages 31/64 of it at 256 slots (five eighths below): 54 KB a block and registers
+//    held to 168 put three blocks on a CU, where the whole budget (105 KB) leaves one, a single
+//    wave per SIMD: 1537 -> 926 us on the 3.0 M two-phase dam break.  With WIDE it takes the whole
+//    budget, for cases whose tiles would not fit otherwise (pair_wide, which decides on the
+//    particles of a sub-cell) and would read their candidates from global memory.
+template <class Pol, int BLOCK, bool WIDE>
 struct PairCap {
-  static constexpr int value = Pol::MIXED ? plan_cap(BLOCK) * 5 / 8 : plan_cap(BLOCK);
+  static constexpr int value = WIDE                          ? plan_cap(BLOCK)
+                               : Pol::MIXED || BLOCK < 256   ? plan_cap(BLOCK) * 5 / 8
+                                                             : plan_cap(BLOCK) * 31 / 64;
 };
+// Whether a P64 pair kernel of BLOCK slots takes the whole budget: a band tile has about BLOCK lanes
+// over BLOCK / (2 q) sub-rows of two sub-columns, q the particles of a sub-cell, and stages six
+// sub-columns over those rows and up to 6 more, 3 BLOCK + 36 q candidates, here with 5% to spare.
+// At h/d = 1.3 (q = 4.0) that is 959 of 992 at 256 slots; past q = 4.9 the whole budget is taken.
+inline bool pair_wide(int B, double q) {
+  const int cap = B < 256 ? plan_cap(B) * 5 / 8 : plan_cap(B) * 31 / 64;
+  return 1.05 * (3.0 * B + 36.0 * q) > cap;
+}
 // The shift stages three quarters of the pair's budget: tiles over both sub-columns of a cell
 // column stage about 3.4 candidates a lane (a dense 256-lane tile ~870), and the smaller LDS
 // lets 8 blocks of 256 share a CU.
@@ -1536,12 +1572,13 @@ struct ShiftCap {
 // src/fluid.cu:429-440) and advances every particle's path length since the hash.  With
 // record (the shift runs on the same tiles), it also records the shift passes' candidate runs
 // (f_wc, tile_d0) from its windows widened by the skin.
-template <class Pol, bool VISCID, int BLOCK>
-__global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : 1))
+template <class Pol, bool VISCID, int BLOCK, bool WIDE>
+__global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
     k_fluid_pair_update(Dev<Pol> d, const TilePlan *plans, const int *ntiles, int record) {
+#pragma clang fp contract(off)
   using R = typename Pol::R;
   using R2 = typename V2<R>::T;
-  constexpr int CAP = PairCap<Pol, BLOCK>::value;
+  constexpr int CAP = PairCap<Pol, BLOCK, WIDE>::value;
   // walls of the tile's 3x3 cell columns over its cell rows follow the fluid candidates
   // (a tile's fluid candidates rarely fill CAP: the walls use what they leave, so that the
   // block stays within a fifth of the CU's LDS at 128 slots)
@@ -1604,8 +1641,8 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : 1))
         },
         [&](int l, const Ld &v, int) {
           if constexpr (Pol::MIXED)  // tile frame
-            s_pos[l] = R2{v.pos.x + (float)((cxy_x(v.pk) >> 1) - gcx) * fdx,
-                          v.pos.y + (float)((cxy_y(v.pk) >> 1) - gcy) * fdy};
+            s_pos[l] = R2{kfma((float)((cxy_x(v.pk) >> 1) - gcx), fdx, v.pos.x),
+                          kfma((float)((cxy_y(v.pk) >> 1) - gcy), fdy, v.pos.y)};
           else
             s_pos[l] = v.pos;
           s_vel[l] = v.vel;
@@ -1632,7 +1669,7 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : 1))
       const int phj = ld32(d.w_phase, g);
       if constexpr (Pol::MIXED) {  // tile frame
         const int wk = ld32(d.w_cxy, g);
-        s_pos[l] = R2{wx + (float)(cxy_x(wk) - P.cx) * fdx, wy + (float)(cxy_y(wk) - P.cy_ref) * fdy};
+        s_pos[l] = R2{kfma((float)(cxy_x(wk) - P.cx), fdx, wx), kfma((float)(cxy_y(wk) - P.cy_ref), fdy, wy)};
       } else {
         s_pos[l] = R2{wx, wy};
       }
@@ -1660,8 +1697,9 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : 1))
     else
       lp = lane_pos(x0, y0, lsx, sy, cp);
     const bool liq = phi == 0;
-    const R cs = cp.c[phi], csinv = cp.cinv[phi], mu8 = cp.mu8[phi];
-    const R rhoi_inv = krcp<R>(rhoi);
+    const R cs = cp.c[phi], csinv = cp.cinv[phi], hmu = R(0.5) * cp.mu8[phi];
+    // the phases whose neighbours a lane's colour leaves out: gas (1) for liquid lanes, else none
+    const int col_skip = liq ? 1 : -1;
     const LoopConsts<R> K(cp);
     const R eps_h2 = cp.eps_h2, qrc2 = cp.quarter_rc2;
     // LDS index of the lane's own slot (in the span of its sub-column)
@@ -1673,23 +1711,24 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : 1))
     }
     PairSums<R> S;
     // fluidFluidCalculate on one candidate (w = 0 outside the cut-off: exact zero terms);
-    // INSIDE: the candidate is known to lie inside the cut-off.  The reference's sticky near
-    // flag (src/fluid.cu:67-73) ends at HAS_NEAR (2) if a FREE_SURFACE neighbour lies within
-    // half the cut-off, else HAS (1) if one lies within it: the smallest such r^2 decides.
+    // INSIDE: the candidate is known to lie inside the cut-off and is not the lane itself.  The
+    // reference's sticky near flag (src/fluid.cu:67-73) ends at HAS_NEAR (2) if a FREE_SURFACE
+    // neighbour lies within half the cut-off, else HAS (1) if one lies within it: the smallest
+    // such r^2 decides.
     auto fluid_j = [&](auto inside, bool self, R dx, R dy, R r2, R uj, R vj, R rhoj, R pj, int fl, bool in) {
       constexpr bool INSIDE = decltype(inside)::value;
       R w;
-      bool fs = liq & !self & ((fl >> 4) == 1);
+      bool fs = (fl >> 4) == 1;
       if constexpr (INSIDE) {
-        w = K.w_in(r2);
+        w = K.gauss_in(r2);
       } else {
-        const R wk = K.w(r2);
+        const R wk = K.gauss(r2);
         w = in ? wk : R(0);
-        fs = fs & in & (r2 < K.rc2);
+        fs = fs & in & !self & (r2 < K.rc2);
       }
-      riemann_pair<R, VISCID>(dx, dy, r2, w, ui, vi, uj, vj, rhoi, rhoi_inv, rhoj, pi, pj, cs, csinv, mu8, eps_h2, S);
-      if (!(liq && (fl & 0xf) == 1)) S.col += r2 * w;
-      S.fsr = (fs && r2 < S.fsr) ? r2 : S.fsr;
+      riemann_pair<R, VISCID>(dx, dy, r2, w, ui, vi, uj, vj, rhoi, rhoj, pi, pj, cs, csinv, hmu, eps_h2, S);
+      S.col = kfma(r2, (fl & 0xf) == col_skip ? R(0) : w, S.col);
+      S.fsr = fmin(S.fsr, fs ? r2 : R(1e30));
     };
     using Cut = std::false_type;
     using Inside = std::true_type;
@@ -1700,7 +1739,7 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : 1))
     auto rows = [&](int sc, int qa, int qb, R bx, R by) {  // global memory
       for_range<2>(lbc[sc * ny21 + qa], lbc[sc * ny21 + qb + 1], [&](int s) {
         const R dx = A.vx[s] - bx, dy = A.vy[s] - by;
-        fluid_j(Cut{}, s == i, dx, dy, dx * dx + dy * dy, A.vu[s], A.vv[s], A.vrho[s], A.p[s],
+        fluid_j(Cut{}, s == i, dx, dy, norm2(dx, dy), A.vu[s], A.vv[s], A.vrho[s], A.p[s],
                 (int)d.f_phase[s] | ((int)d.f_cls[s] << 4), true);
       });
     };
@@ -1712,11 +1751,11 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : 1))
       if (!staged) d.f_wc[i] = uint4{0u, 0u, 0u, 0u};
     }
     // the lane in the tile frame (M32 staged positions are re-based on it)
-    const R yg = Pol::MIXED ? yi + (R)(cy - P.cy_ref) * cp.cdy_r : yi;
+    const R yg = Pol::MIXED ? kfma((R)(cy - P.cy_ref), cp.cdy_r, yi) : yi;
     auto staged_j = [&](auto inside, int l, bool in) {
       const R2 pj = s_pos[l], vj = s_vel[l], rp = s_rp[l];
       const R dx = pj.x - xi, dy = pj.y - yg;
-      fluid_j(inside, l == own, dx, dy, dx * dx + dy * dy, vj.x, vj.y, rp.x, rp.y, s_fl[l], in);
+      fluid_j(inside, l == own, dx, dy, norm2(dx, dy), vj.x, vj.y, rp.x, rp.y, s_fl[l], in);
     };
     if (staged) {
       // staged windows (one run each): first mark the candidates inside the cut-off (32-bit
@@ -1743,7 +1782,7 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : 1))
         // once, so that the bit positions cost no instruction per candidate
         auto r2of = [&](const R2 &pj) {
           const R dx = pj.x - xi, dy = pj.y - yg;
-          return dx * dx + dy * dy;
+          return norm2(dx, dy);
         };
         const R rc2 = K.rc2;
         unsigned m = 0u;
@@ -1788,7 +1827,7 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : 1))
         };
         auto use = [&](const Cand &q) {
           const R dx = q.p.x - xi, dy = q.p.y - yg;
-          fluid_j(Inside{}, q.l == own, dx, dy, dx * dx + dy * dy, q.v.x, q.v.y, q.r.x, q.r.y, q.fl, true);
+          fluid_j(Inside{}, false, dx, dy, norm2(dx, dy), q.v.x, q.v.y, q.r.x, q.r.y, q.fl, true);
         };
         Cand cur = next();
         // unrolled by two, so that every other round reads into the registers the previous one
@@ -1834,6 +1873,9 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : 1))
         } else {
           mk[q] = mark(std::false_type{}, s0, s1, ms);
         }
+        // the lane itself (in the window of its own sub-column): no term, and no FREE_SURFACE
+        // neighbour of its own
+        if (o == 0 && own >= s0 && own < s1) mk[q] &= ~(1u << (own - s0));
       }
       if (record) d.f_wc[i] = rr.entry(cum0);
       // windows in the order 0, -1, +1, ... (those at -k and +k in one loop unless one of them
@@ -1890,13 +1932,13 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : 1))
         const int2 rw = d.w_range[cp.cell_off + jx * cp.ny + jy];
         for_range<4>(rw.x, rw.y, [&](int s) {  // fluidVirtCalculate: rho_j = rho0[wall phase]
           const R dx = ld32(d.w_vx, s) - bx, dy = ld32(d.w_vy, s) - by;
-          const R r2 = dx * dx + dy * dy;
+          const R r2 = norm2(dx, dy);
           if (!(r2 < K.rc2)) return;
-          const R w = K.w(r2);
+          const R w = K.gauss_in(r2);
           const int phj = d.w_phase[s];
-          riemann_pair<R, VISCID>(dx, dy, r2, w, ui, vi, d.w_u[s], d.w_v[s], rhoi, rhoi_inv, cp.rho0[phj], pi,
-                                  d.w_p[s], cs, csinv, mu8, eps_h2, S);
-          if (!(liq && phj == 1)) S.col += r2 * w;
+          riemann_pair<R, VISCID>(dx, dy, r2, w, ui, vi, d.w_u[s], d.w_v[s], rhoi, cp.rho0[phj], pi, d.w_p[s], cs,
+                                  csinv, hmu, eps_h2, S);
+          S.col = kfma(r2, phj == col_skip ? R(0) : w, S.col);
         });
       }
     }
@@ -1912,16 +1954,17 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : 1))
         for_range<2>(rs.x, rs.y, [&](int k) {  // fluidSolidCalculate: rho_j = rho_i
           const int j = d.s_sorted[k];
           const R dx = d.s_vx[j] - bx, dy = d.s_vy[j] - by;
-          const R r2 = dx * dx + dy * dy;
+          const R r2 = norm2(dx, dy);
           if (!(r2 < K.rc2)) return;
-          const R w = K.w(r2);
-          riemann_pair<R, VISCID>(dx, dy, r2, w, ui, vi, (R)d.su[j], (R)d.sv[j], rhoi, rhoi_inv, rhoi, pi, d.s_p[j],
-                                  cs, csinv, mu8, eps_h2, S);
+          const R w = K.gauss_in(r2);
+          riemann_pair<R, VISCID>(dx, dy, r2, w, ui, vi, (R)d.su[j], (R)d.sv[j], rhoi, rhoi, pi, d.s_p[j], cs, csinv,
+                                  hmu, eps_h2, S);
         });
       }
     }
+    pair_finish(S, rhoi, K.kdc);
     d.f_col[i] = S.col;
-    const int near = S.fsr < qrc2 ? 2 : (S.fsr < K.rc2 ? 1 : 0);
+    const int near = !liq ? 0 : S.fsr < qrc2 ? 2 : (S.fsr < K.rc2 ? 1 : 0);
     d.f_near[i] = (int8_t)near;
     // the fluid class of this step (correctionUpdate, src/fluid.cu:369-427), a function of
     // phase, colour and near flag only; it is set only where the case shifts
@@ -1942,16 +1985,16 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : 1))
     // fluidUpdate, integrated in double
     double ax = (double)S.ax, ay = (double)S.ay;
     if (cp.steady) {
-      ax += -0.1 * u0;
-      ay += -0.1 * v0;
+      ax = kfma(-0.1, u0, ax);
+      ay = kfma(-0.1, v0, ay);
     }
     const double dt = d.dtv[c];
-    double x = x0 + u0 * dt, y = y0 + v0 * dt;
-    const double u = u0 + (ax + cp.gx_d) * dt, v = v0 + (ay + cp.gy_d) * dt;
-    double rho = r0 + (double)S.drho * dt;
+    double x = kfma(u0, dt, x0), y = kfma(v0, dt, y0);
+    const double u = kfma(ax + cp.gx_d, dt, u0), v = kfma(ay + cp.gy_d, dt, v0);
+    double rho = kfma((double)S.drho, dt, r0);
     rho = fmax(rho, cp.rho_min_d[phi]);
     // densityToPressure (src/fluid.cu:15-23)
-    const double p = fmax((pow(rho * cp.rho0_inv_d[phi], cp.gam_d[phi]) - 1.0) * cp.rho2p_d[phi] + cp.p_bg_d,
+    const double p = fmax(kfma(pow(rho * cp.rho0_inv_d[phi], cp.gam_d[phi]) - 1.0, cp.rho2p_d[phi], cp.p_bg_d),
                           cp.p_min_d);
     x = fmin(fmax(x, cp.dxmin), cp.dxmax);
     y = fmin(fmax(y, cp.dymin), cp.dymax);
@@ -1969,10 +2012,10 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : 1))
       B.vv[i] = (float)v;
       B.vrho[i] = (float)rho;
     }
-    const double u2 = u * u + v * v;
+    const double u2 = norm2(u, v);
     my_u2 = (unsigned long long)__double_as_longlong(u2);
     const double mx = x - x0, my = y - y0;
-    B.cum[i] = (float)((double)cum0 + sqrt(mx * mx + my * my));
+    B.cum[i] = (float)((double)cum0 + sqrt(norm2(mx, my)));
     if (isnan(rho) || isnan(x) || isnan(y) || isnan(u2)) atomicOr(d.status, kStNaN);
   }
   // per-case max |u|^2 (non-negative doubles order like their bit patterns)
@@ -2050,6 +2093,7 @@ __device__ __forceinline__ void shift_tile(const Dev<Pol> &d, const TilePlan &P,
                                            const LB (*s_lb)[TileRows<BLOCK>::value + 1], const int (*s_wlb)[WROWS + 1],
                                            float D, float Dsp, bool runs, bool staged, bool wstaged,
                                            const WallSpans &W) {
+#pragma clang fp contract(off)
   using R = typename Pol::R;
   using R2 = typename V2<R>::T;
   const int t = threadIdx.x, c = P.c;
@@ -2082,10 +2126,10 @@ __device__ __forceinline__ void shift_tile(const Dev<Pol> &d, const TilePlan &P,
     lp = lane_pos(x0, y0, lsx, sy, cp);
   const LoopConsts<R> K(cp);
   R gx = 0, gy = 0;
-  auto add = [&](R dx, R dy) {
-    const R w = K.w(dx * dx + dy * dy);
-    gx += dx * w;
-    gy += dy * w;
+  auto add = [&](R dx, R dy) {  // (kd c32 multiplies the sums, below)
+    const R w = K.gauss(norm2(dx, dy));
+    gx = kfma(dx, w, gx);
+    gy = kfma(dy, w, gy);
   };
   const float Rp = prune_radius(cp, staged, D) + ((MODE == kShiftRecord && staged) ? cp.skin_grow : 0.f);
   const int *lbc = d.f_lb + cp.lb_off;
@@ -2105,16 +2149,16 @@ __device__ __forceinline__ void shift_tile(const Dev<Pol> &d, const TilePlan &P,
   // one staged candidate (fluid or wall); w = 0 outside the cut-off; returns r^2 (scaled)
   auto staged_term = [&](int l) {
     const R2 pj = s_pos[l];
-    const R dx = pj.x - xs, dy = pj.y - ys, r2 = dx * dx + dy * dy;
+    const R dx = pj.x - xs, dy = pj.y - ys, r2 = norm2(dx, dy);
     if constexpr (Pol::MIXED) {
       const R e = __builtin_amdgcn_exp2f(-r2);
       const R w = r2 < rc2s ? e : R(0);
-      gxs += dx * w;
-      gys += dy * w;
+      gxs = kfma(dx, w, gxs);
+      gys = kfma(dy, w, gys);
     } else {
-      const R w = K.w(r2);
-      gx += dx * w;
-      gy += dy * w;
+      const R w = K.gauss(r2);
+      gx = kfma(dx, w, gx);
+      gy = kfma(dy, w, gy);
     }
     return r2;
   };
@@ -2219,9 +2263,11 @@ __device__ __forceinline__ void shift_tile(const Dev<Pol> &d, const TilePlan &P,
       });
     }
   }
+  gx *= K.kdc;
+  gy *= K.kdc;
   if constexpr (Pol::MIXED) {
-    gx += gxs * cp.kdc_s;
-    gy += gys * cp.kdc_s;
+    gx = kfma(gxs, cp.kdc_s, gx);
+    gy = kfma(gys, cp.kdc_s, gy);
   }
   const R umax = d.umax[c];
   const R shift_k = (R)(cp.shift_ch * d.dtv[c]);  // particle_shift_coef h dt
@@ -2232,18 +2278,18 @@ __device__ __forceinline__ void shift_tile(const Dev<Pol> &d, const TilePlan &P,
     syv = 0;
   } else if (cls == 1 || cls == 2) {  // FREE_SURFACE / VICINITY: tangential part only
     R nx = 0, ny = 0;
-    const R g2 = gx * gx + gy * gy;
+    const R g2 = norm2(gx, gy);
     if (g2 > R(0)) {
       const R ig = krsqrt<R>(g2);
       nx = gx * ig;
       ny = gy * ig;
     }
-    if (sqrt(nx * nx + ny * ny) < R(0.1)) {
+    if (sqrt(norm2(nx, ny)) < R(0.1)) {
       nx = 0;
       ny = 0;
     }
-    sxv = (R(1) - nx * nx) * dxs - nx * ny * dys;
-    syv = -ny * nx * dxs + (R(1) - ny * ny) * dys;
+    sxv = kfma(kfma(-nx, nx, R(1)), dxs, -((nx * ny) * dys));
+    syv = kfma(kfma(-ny, ny, R(1)), dys, -((ny * nx) * dxs));
   }
   sxv *= umax;
   syv *= umax;
@@ -2266,7 +2312,7 @@ __device__ __forceinline__ void shift_tile(const Dev<Pol> &d, const TilePlan &P,
   }
   // path length: this pass moved the particle by (sxv, syv); the passes after a recording
   // one count from it and the last adds the path since the hash it recorded
-  const float sx2 = (float)sxv, sy2 = (float)syv, step = __builtin_amdgcn_sqrtf(sx2 * sx2 + sy2 * sy2);
+  const float sx2 = (float)sxv, sy2 = (float)syv, step = __builtin_amdgcn_sqrtf(norm2(sx2, sy2));
   if constexpr (MODE == kShiftPlain)
     B.cum[i] = cum0 + step;
   else if constexpr (MODE == kShiftRecord)
@@ -2279,8 +2325,8 @@ __device__ __forceinline__ void shift_tile(const Dev<Pol> &d, const TilePlan &P,
       A.y[i] = y;
     }
     const R *L = d.f_L + 4 * i;
-    A.u[i] += (double)(L[0] * sn.x + L[1] * sn.y);
-    A.v[i] += (double)(L[2] * sn.x + L[3] * sn.y);
+    A.u[i] += (double)kfma(L[0], sn.x, L[1] * sn.y);
+    A.v[i] += (double)kfma(L[2], sn.x, L[3] * sn.y);
   } else {
     d.f_sacc[2 * i] = sn.x;
     d.f_sacc[2 * i + 1] = sn.y;
@@ -2335,7 +2381,7 @@ __global__ void __launch_bounds__(BLOCK, (MODE == kShiftCached ? 8 : 7))
         },
         [&](int l, const Ld &v, int) {
           if constexpr (Pol::MIXED)  // tile frame, scaled units
-            s_pos[l] = R2{fmaf(v.pos.x, gs, xo), (v.pos.y + (float)(((v.pk & 0xffff) >> 1) - gcy) * fdy) * gs};
+            s_pos[l] = R2{kfma(v.pos.x, gs, xo), kfma((float)(((v.pk & 0xffff) >> 1) - gcy), fdy, v.pos.y) * gs};
           else
             s_pos[l] = v.pos;
           dmax = max(dmax, v.cum);
@@ -2352,7 +2398,7 @@ __global__ void __launch_bounds__(BLOCK, (MODE == kShiftCached ? 8 : 7))
       const R wx = ld32(d.w_vx, g), wy = ld32(d.w_vy, g);
       if constexpr (Pol::MIXED) {  // tile frame, scaled units
         const int wk = ld32(d.w_cxy, g);
-        s_pos[l] = R2{(wx + (float)(cxy_x(wk) - P.cx) * fdx) * gs, (wy + (float)(cxy_y(wk) - P.cy_ref) * fdy) * gs};
+        s_pos[l] = R2{kfma((float)(cxy_x(wk) - P.cx), fdx, wx) * gs, kfma((float)(cxy_y(wk) - P.cy_ref), fdy, wy) * gs};
       } else {
         s_pos[l] = R2{wx, wy};
       }
@@ -2434,7 +2480,7 @@ __device__ __forceinline__ void solid_couple_block(const Dev<Pol> &d, int bid) {
     const int pk = d.s_cxy[i], cx = cxy_x(pk), cy = cxy_y(pk);
     const R xi = d.s_vx[i], yi = d.s_vy[i];
     const LoopConsts<R> K(cp);
-    const R eR = cp.eR, k2c = cp.k2c, hinv2 = cp.hinv2;
+    const R eR = cp.eR, k2c = cp.k2c, nhl2 = cp.nhl2;
     const auto &F = d.fa;
     // fluid: the 3x3 cells' 18 runs spread over the group's lanes (as in the force kernel)
     for (int r = l; r < kCellRuns; r += kSolidLanes) {
@@ -2445,7 +2491,7 @@ __device__ __forceinline__ void solid_couple_block(const Dev<Pol> &d, int bid) {
         const R dx = f.x - bx, dy = f.y - by;
         const R r2 = dx * dx + dy * dy;
         if (r2 < K.rc2) {
-          const R w = (kexp<R>(-(r2 * hinv2)) - eR) * k2c;
+          const R w = (kgauss<R>(r2, nhl2) - eR) * k2c;
           S += w;
           P += f.p * w;
         }

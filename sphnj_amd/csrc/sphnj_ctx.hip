@@ -183,6 +183,7 @@ struct Engine : EngineBase {
   int max_tiles(int B) const { return kMaxPieces * (nblk(d.nf, B) + G); }
   int grid_tiles(int B) const { return (max_tiles(B) + kXcds - 1) / kXcds * kXcds; }
   bool viscid = false;
+  double sub_particles = 0.0;  // particles of a full sub-cell, the most over the cases with fluid
   // the persistent solid kernel: barrier words and the grid (0 = the device cannot hold the
   // solids' blocks resident at half its capacity: the sub-steps fall back to 2 S launches)
   GridSync gsync{};
@@ -245,7 +246,6 @@ struct Engine : EngineBase {
     std::memset(&c, 0, sizeof(c));
     c.rc2 = (R)D.rc2;
     c.quarter_rc2 = (R)(0.25 * D.rc2);
-    c.hinv2 = (R)D.hinv2;
     c.nhl2 = (R)(-D.hinv2 * 1.4426950408889634);
     c.kdc = (R)D.kdc;
     {
@@ -362,6 +362,8 @@ struct Engine : EngineBase {
       fill_case(D[c], hc[c]);
       if (!St[c].sx.empty()) hc[c].dt_solid_cap = D[c].dt_solid_cap;
       viscid = viscid || D[c].viscid;
+      if (!St[c].fx.empty())
+        sub_particles = std::max(sub_particles, 0.25 * D[c].cdx * D[c].cdy / (D[c].d * D[c].d));
       hc[c].cell_off = total_cells;
       total_cells += hc[c].ncell;
       hc[c].col_off = G;
@@ -807,15 +809,25 @@ struct Engine : EngineBase {
     return SPHNJ_OK;
   }
 
-  template <int B>
-  void pair_at() {
+  template <int B, bool WIDE>
+  void pair_launch() {
     const int b = bidx(B);
     const int *nt = tile_off[b] + G;
     const int rec = pair_rec ? 1 : 0;
     if (viscid)
-      k_fluid_pair_update<Pol, true, B><<<grid_tiles(B), B, 0, stream>>>(d, plans[b], nt, rec);
+      k_fluid_pair_update<Pol, true, B, WIDE><<<grid_tiles(B), B, 0, stream>>>(d, plans[b], nt, rec);
     else
-      k_fluid_pair_update<Pol, false, B><<<grid_tiles(B), B, 0, stream>>>(d, plans[b], nt, rec);
+      k_fluid_pair_update<Pol, false, B, WIDE><<<grid_tiles(B), B, 0, stream>>>(d, plans[b], nt, rec);
+  }
+  template <int B>
+  void pair_at() {
+    if constexpr (!Pol::MIXED) {
+      if (pair_wide(B, sub_particles)) {
+        pair_launch<B, true>();
+        return;
+      }
+    }
+    pair_launch<B, false>();
   }
   int launch_pair(int blk) {
     int rc;
