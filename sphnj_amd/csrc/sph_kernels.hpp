@@ -3002,6 +3002,41 @@ __global__ void __launch_bounds__(256) k_ref_fill(Dev<Pol> d, const int *cxy, co
   }
 }
 
+// ---- download: the fields of one species of one case in input order -------------------------
+// A field of `bytes` (1, 4, 8, 16 or 32) per particle, from its slot array to dst in input order.
+struct GatherField {
+  const char *src;
+  char *dst;
+  int bytes;
+};
+constexpr int kGatherMax = 14;
+struct GatherArgs {
+  GatherField f[kGatherMax];
+  int nf, n, lo;    // fields, particles, the case's first slot
+  const int *orig;  // slot -> global original index (null: slots are in input order)
+};
+// A thread per slot: slots in order read whole lines, and slots that are neighbours in space have
+// original indices near each other, so the scattered writes of a wave meet in L2.
+__global__ void __launch_bounds__(256) k_gather(GatherArgs a) {
+  const int i = blockIdx.x * 256 + (int)threadIdx.x;
+  if (i >= a.n) return;
+  const int s = a.lo + i, o = a.orig ? a.orig[s] - a.lo : i;
+  for (int k = 0; k < a.nf; ++k) {
+    const GatherField f = a.f[k];
+    if (f.bytes == 8)
+      reinterpret_cast<int2 *>(f.dst)[o] = reinterpret_cast<const int2 *>(f.src)[s];
+    else if (f.bytes == 4)
+      reinterpret_cast<int *>(f.dst)[o] = reinterpret_cast<const int *>(f.src)[s];
+    else if (f.bytes == 16)
+      reinterpret_cast<int4 *>(f.dst)[o] = reinterpret_cast<const int4 *>(f.src)[s];
+    else if (f.bytes == 32) {
+      reinterpret_cast<int4 *>(f.dst)[2 * (size_t)o] = reinterpret_cast<const int4 *>(f.src)[2 * (size_t)s];
+      reinterpret_cast<int4 *>(f.dst)[2 * (size_t)o + 1] = reinterpret_cast<const int4 *>(f.src)[2 * (size_t)s + 1];
+    } else
+      f.dst[o] = f.src[s];
+  }
+}
+
 // ---- inspection: neighbour lists of the fluid particles ---------------------------------
 template <class Pol>
 __global__ void __launch_bounds__(256) k_neighbors(Dev<Pol> d, int lo, int hi, const int *offset, int *count,
