@@ -25,7 +25,7 @@ struct M32 {
 template <class R>
 struct CaseDev {
   // kernel (Kernel::initiate, src/kernel.cpp:25-41)
-  R rc2, kdc, k2c, eR, h, eps_h2;  // eps_h2 = 0.01 h^2
+  R rc2, hinv2, kdc, k2c, eR, h, eps_h2;  // eps_h2 = 0.01 h^2
   R nhl2;  // -log2(e) / h^2: exp(-r^2/h^2) = 2^(r^2 nhl2)
   // scaled units of the M32 shift loop: x' = x sqrt(hinv2 log2 e), so exp(-r^2/h^2) = 2^-r'^2
   float gscale, rc2s, kdc_s;  // scale, rc^2 scaled, kd c32 / scale
@@ -260,6 +260,15 @@ __device__ __forceinline__ double kgauss<double>(double r2, double nhl2) {
 template <>
 __device__ __forceinline__ float kgauss<float>(float r2, float nhl2) {
   return __builtin_amdgcn_exp2f(r2 * nhl2);
+}
+
+// The same where M32 has always scaled by 1/h^2 and by log2(e) apart (walls, coupling).
+template <class R>
+__device__ __forceinline__ R kgauss2(R r2, R hinv2, R nhl2) {
+  if constexpr (sizeof(R) == 4)
+    return __builtin_amdgcn_exp2f(-(r2 * hinv2) * 1.4426950408889634f);
+  else
+    return kgauss<R>(r2, nhl2);
 }
 
 // 1/sqrt(x) and 1/x.  FP64: the hardware's estimate y (relative error e/2 or e, about 2^-23) and

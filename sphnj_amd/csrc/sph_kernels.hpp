@@ -528,7 +528,7 @@ __global__ void __launch_bounds__(256) k_wall_normal(Dev<Pol> d) {
         const R dx = d.w_vx[s] - bx, dy = d.w_vy[s] - by;
         const R r2 = dx * dx + dy * dy;
         if (r2 < cp.rc2) {
-          const R w = kgauss<R>(r2, cp.nhl2) * cp.kdc;
+          const R w = kgauss2<R>(r2, cp.hinv2, cp.nhl2) * cp.kdc;
           nx -= dx * w;
           ny -= dy * w;
         }
@@ -584,7 +584,7 @@ __device__ __forceinline__ void wall_update_block(const Dev<Pol> &d, int bid) {
           const R dx = F.vx[s] - bx, dy = F.vy[s] - by;
           const R r2 = dx * dx + dy * dy;
           if (!(r2 < cp.rc2)) continue;
-          const R w = (kgauss<R>(r2, cp.nhl2) - cp.eR) * cp.k2c;
+          const R w = (kgauss2<R>(r2, cp.hinv2, cp.nhl2) - cp.eR) * cp.k2c;
           S[j] += w;
           U[j] += F.vu[s] * w;
           V[j] += F.vv[s] * w;
@@ -1456,37 +1456,24 @@ struct LoopConsts {
     const R e = kgauss<R>(r2, nhl2);
     return r2 < rc2 ? e : R(0);
   }
-  // the same of a candidate known to lie inside the cut-off
-  __device__ __forceinline__ R gauss_in(R r2) const { return kgauss<R>(r2, nhl2); }
-  // gradient weight w'(r^2) = exp(-r^2/h^2) kd c32, 0 outside the cut-off
-  __device__ __forceinline__ R w(R r2) const { return gauss(r2) * kdc; }
+  // gradient weight w'(r^2) = exp(-r^2/h^2) kd c32 of a candidate known to lie inside the cut-off
+  __device__ __forceinline__ R w_in(R r2) const { return kgauss<R>(r2, nhl2) * kdc; }
+  // the same, 0 outside the cut-off
+  __device__ __forceinline__ R w(R r2) const {
+    const R e = w_in(r2);
+    return r2 < rc2 ? e : R(0);
+  }
 };
 
 // ======================================================================================
 // FLUID: Riemann pair loop fused with the explicit update
 // ======================================================================================
 
-// Sums over a lane's neighbours, with the factors that a lane's terms share left out (pair_finish
-// multiplies them in once): ax, ay without -2 kd c32 / rho_i, drho without 2 kd c32, L without
-// -kd c32 and col without kd c32.
 template <class R>
 struct PairSums {
   R ax = 0, ay = 0, drho = 0, L00 = 0, L01 = 0, L10 = 0, L11 = 0, col = 0;
   R fsr = R(1e30);  // smallest r^2 of a FREE_SURFACE neighbour inside the cut-off
 };
-template <class R>
-__device__ __forceinline__ void pair_finish(PairSums<R> &A, R rhoi, R kdc) {
-#pragma clang fp contract(off)
-  const R s = (R(-2) * kdc) * krcp<R>(rhoi);
-  A.ax *= s;
-  A.ay *= s;
-  A.drho *= R(2) * kdc;
-  A.L00 *= -kdc;
-  A.L01 *= -kdc;
-  A.L10 *= -kdc;
-  A.L11 *= -kdc;
-  A.col *= kdc;
-}
 
 template <class R>
 __device__ __forceinline__ R norm2(R dx, R dy) {
@@ -1494,43 +1481,88 @@ __device__ __forceinline__ R norm2(R dx, R dy) {
   return kfma(dx, dx, dy * dy);
 }
 
+// What a lane's Riemann terms share.
+template <class R>
+struct PairLane {
+  R u, v, rho, p, c, cinv;
+  R mu8, rho_inv, m2_rho_inv, rho2, p_cinv;  // 8 mu; 1 / rho_i, -2 / rho_i, 2 rho_i, p_i / c_i (M32)
+  R eps_h2;
+  __device__ __forceinline__ PairLane(R u_, R v_, R rho_, R p_, R c_, R cinv_, R mu8_, R eps)
+      : u(u_), v(v_), rho(rho_), p(p_), c(c_), cinv(cinv_), mu8(mu8_), eps_h2(eps) {
+    rho_inv = krcp<R>(rho);
+    m2_rho_inv = R(-2) * rho_inv;
+    rho2 = R(2) * rho;
+    p_cinv = p * cinv;
+  }
+};
+
 // Riemann terms of fluidFluidCalculate / fluidSolidCalculate / fluidVirtCalculate
-// (src/fluid.cu:25-191), with the algebra rearranged around q = (u_i - u_j).dx, d = p_j - p_i and
-// a = rho_i / (rho_i + rho_j):
-//   du = q / r,  p* = p_i + a d + a rho_j max(du, 0) min(3 du, c_i),
-//   (u_i - v*).dx = (rho_j q + d r / c_i) / (rho_i + rho_j),
-// and w = exp(-r^2/h^2) (0 outside the cut-off), so that every factor a lane's terms share comes
-// in once, in pair_finish.  d is formed first: equal pressures give exact zeros.  r^2 is kept off 0
-// for the root only; at r = 0 every term is 0 through dx, dy and q.  These terms are more than half
-// of the pair kernel's vector instructions, which is what bounds it: 121 per two candidates with
-// their fetch, against 136 with the density weights of both sides, the lane's factors in every
-// term and a test for r = 0.  464 -> 437 us a launch on the 3.0 M two-phase dam break (M32),
-// 922 -> 866 us (P64).
+// (src/fluid.cu:25-191), with the algebra rearranged around q = (u_i - u_j).dx:
+//   du = q / r,  (u_i - v*).dx = rho_j q / (rho_i + rho_j) - (p_i - p_j) r / ((rho_i + rho_j) c).
+// w = w'(r^2), 0 outside the cut-off.  r^2 is kept off 0 for the root only: at r = 0 every term is 0
+// through dx, dy and q; max(du, 0) takes the place of the test for an approaching pair.
 // Every multiply-add is written out and contraction is off: what a lane sums must not depend on
 // how the compiler happens to fuse an instance of the kernel (block sizes, staged or global
 // candidates), and does not.
-template <class R, bool VISCID>
-__device__ __forceinline__ void riemann_pair(R dx, R dy, R r2, R w, R ui, R vi, R uj, R vj, R rhoi, R rhoj, R pi, R pj,
-                                             R cs, R csinv, R hmu, R eps_h2, PairSums<R> &A) {
+// M32 keeps the roundings of the separate density weights and lane factors: the classes of particles
+// at the interface hang on thresholds that a last bit can cross.  P64 forms p* from d = p_j - p_i and
+// leaves the factors of particle i to the sums (pair_finish): fewer FP64 instructions, 922 -> 874 us
+// a launch on the 3.0 M two-phase dam break.
+// (PI_FUSED: of M32's two products in p*, p_i's is the fused one; the walls of a tile that does not
+// stage them.)
+template <class R, bool VISCID, bool PI_FUSED = false>
+__device__ __forceinline__ void riemann_pair(R dx, R dy, R r2, R q, R w, R du_, R dv_, R rhoj, R pj,
+                                             const PairLane<R> &I, PairSums<R> &A) {
 #pragma clang fp contract(off)
   const R inv_r = krsqrt<R>(fmax(r2, sizeof(R) == 4 ? R(1e-36) : R(1e-290)));
   const R rn = r2 * inv_r;  // |dx|
-  const R du_ = ui - uj, dv_ = vi - vj;
-  const R q = kfma(du_, dx, dv_ * dy);
-  const R d = pj - pi;
-  const R a = rhoi * krcp<R>(rhoi + rhoj);
+  const R isum = krcp<R>(I.rho + rhoj);
   const R du = fmax(q * inv_r, R(0));
-  R ps = kfma(a, d, pi);
-  ps = kfma((a * rhoj) * du, fmin(R(3) * du, cs), ps);
-  if constexpr (VISCID) ps = kfma(hmu, kdiv<R>(q, r2 + eps_h2), ps);  // hmu = 4 mu
-  A.drho = kfma(w * a, kfma(d, csinv * rn, rhoj * q), A.drho);
   const R wdx = w * dx, wdy = w * dy;
-  A.ax = kfma(ps, wdx, A.ax);
-  A.ay = kfma(ps, wdy, A.ay);
-  A.L00 = kfma(du_, wdx, A.L00);
-  A.L01 = kfma(du_, wdy, A.L01);
-  A.L10 = kfma(dv_, wdx, A.L10);
-  A.L11 = kfma(dv_, wdy, A.L11);
+  if constexpr (sizeof(R) == 4) {
+    const R ai = I.rho * isum, aj = rhoj * isum;
+    const R ps = kfma((I.rho * aj) * du, fmin(R(3) * du, I.c),
+                      PI_FUSED ? kfma(I.p, aj, pj * ai) : kfma(pj, ai, I.p * aj));
+    const R t = kfma(-I.cinv, pj, I.p_cinv) * isum;
+    const R s = ps * (I.m2_rho_inv * w);
+    A.ax = kfma(s, dx, A.ax);
+    A.ay = kfma(s, dy, A.ay);
+    A.drho = kfma(I.rho2 * w, kfma(q, aj, -(t * rn)), A.drho);
+    if constexpr (VISCID) {
+      const R tv = I.mu8 * kdiv<R>(-q, r2 + I.eps_h2) * I.rho_inv * w;
+      A.ax = kfma(tv, dx, A.ax);
+      A.ay = kfma(tv, dy, A.ay);
+    }
+    A.L00 = kfma(-du_, wdx, A.L00);
+    A.L01 = kfma(-du_, wdy, A.L01);
+    A.L10 = kfma(-dv_, wdx, A.L10);
+    A.L11 = kfma(-dv_, wdy, A.L11);
+  } else {
+    const R d = pj - I.p, a = I.rho * isum;
+    R ps = kfma((a * rhoj) * du, fmin(R(3) * du, I.c), kfma(a, d, I.p));
+    if constexpr (VISCID) ps = kfma(R(0.5) * I.mu8, kdiv<R>(q, r2 + I.eps_h2), ps);
+    A.drho = kfma(w * a, kfma(d, I.cinv * rn, rhoj * q), A.drho);
+    A.ax = kfma(ps, wdx, A.ax);
+    A.ay = kfma(ps, wdy, A.ay);
+    A.L00 = kfma(du_, wdx, A.L00);
+    A.L01 = kfma(du_, wdy, A.L01);
+    A.L10 = kfma(dv_, wdx, A.L10);
+    A.L11 = kfma(dv_, wdy, A.L11);
+  }
+}
+// The factors that the P64 terms leave out.
+template <class R>
+__device__ __forceinline__ void pair_finish(PairSums<R> &A, const PairLane<R> &I) {
+#pragma clang fp contract(off)
+  if constexpr (sizeof(R) == 8) {
+    A.ax *= I.m2_rho_inv;
+    A.ay *= I.m2_rho_inv;
+    A.drho *= R(2);
+    A.L00 = -A.L00;
+    A.L01 = -A.L01;
+    A.L10 = -A.L10;
+    A.L11 = -A.L11;
+  }
 }
 
 // LDS capacity (particles) of a tile of BLOCK slots.  The planner's budget (plan_cap) holds the
@@ -1697,11 +1729,11 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
     else
       lp = lane_pos(x0, y0, lsx, sy, cp);
     const bool liq = phi == 0;
-    const R cs = cp.c[phi], csinv = cp.cinv[phi], hmu = R(0.5) * cp.mu8[phi];
+    const PairLane<R> I(ui, vi, rhoi, pi, cp.c[phi], cp.cinv[phi], cp.mu8[phi], cp.eps_h2);
     // the phases whose neighbours a lane's colour leaves out: gas (1) for liquid lanes, else none
     const int col_skip = liq ? 1 : -1;
     const LoopConsts<R> K(cp);
-    const R eps_h2 = cp.eps_h2, qrc2 = cp.quarter_rc2;
+    const R qrc2 = cp.quarter_rc2;
     // LDS index of the lane's own slot (in the span of its sub-column)
     int own = i;
     if (staged) {
@@ -1715,18 +1747,29 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
     // reference's sticky near flag (src/fluid.cu:67-73) ends at HAS_NEAR (2) if a FREE_SURFACE
     // neighbour lies within half the cut-off, else HAS (1) if one lies within it: the smallest
     // such r^2 decides.
-    auto fluid_j = [&](auto inside, bool self, R dx, R dy, R r2, R uj, R vj, R rhoj, R pj, int fl, bool in) {
+    // swap: r^2 and q with their products in the other order (see eval2).
+    auto fluid_j = [&](auto inside, bool self, bool swap, R dx, R dy, R uj, R vj, R rhoj, R pj, int fl, bool in) {
       constexpr bool INSIDE = decltype(inside)::value;
+      const R du_ = ui - uj, dv_ = vi - vj;
+      R r2, q;
+      if constexpr (Pol::MIXED && INSIDE) {
+        const R a = swap ? dy : dx, b = swap ? dx : dy;
+        r2 = norm2(a, b);
+        q = kfma(swap ? dv_ : du_, a, (swap ? du_ : dv_) * b);
+      } else {
+        r2 = norm2(dx, dy);
+        q = kfma(du_, dx, dv_ * dy);
+      }
       R w;
       bool fs = (fl >> 4) == 1;
       if constexpr (INSIDE) {
-        w = K.gauss_in(r2);
+        w = K.w_in(r2);
       } else {
-        const R wk = K.gauss(r2);
+        const R wk = K.w(r2);
         w = in ? wk : R(0);
         fs = fs & in & !self & (r2 < K.rc2);
       }
-      riemann_pair<R, VISCID>(dx, dy, r2, w, ui, vi, uj, vj, rhoi, rhoj, pi, pj, cs, csinv, hmu, eps_h2, S);
+      riemann_pair<R, VISCID>(dx, dy, r2, q, w, du_, dv_, rhoj, pj, I, S);
       S.col = kfma(r2, (fl & 0xf) == col_skip ? R(0) : w, S.col);
       S.fsr = fmin(S.fsr, fs ? r2 : R(1e30));
     };
@@ -1739,7 +1782,7 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
     auto rows = [&](int sc, int qa, int qb, R bx, R by) {  // global memory
       for_range<2>(lbc[sc * ny21 + qa], lbc[sc * ny21 + qb + 1], [&](int s) {
         const R dx = A.vx[s] - bx, dy = A.vy[s] - by;
-        fluid_j(Cut{}, s == i, dx, dy, norm2(dx, dy), A.vu[s], A.vv[s], A.vrho[s], A.p[s],
+        fluid_j(Cut{}, s == i, false, dx, dy, A.vu[s], A.vv[s], A.vrho[s], A.p[s],
                 (int)d.f_phase[s] | ((int)d.f_cls[s] << 4), true);
       });
     };
@@ -1755,7 +1798,7 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
     auto staged_j = [&](auto inside, int l, bool in) {
       const R2 pj = s_pos[l], vj = s_vel[l], rp = s_rp[l];
       const R dx = pj.x - xi, dy = pj.y - yg;
-      fluid_j(inside, l == own, dx, dy, norm2(dx, dy), vj.x, vj.y, rp.x, rp.y, s_fl[l], in);
+      fluid_j(inside, l == own, false, dx, dy, vj.x, vj.y, rp.x, rp.y, s_fl[l], in);
     };
     if (staged) {
       // staged windows (one run each): first mark the candidates inside the cut-off (32-bit
@@ -1813,9 +1856,11 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
       // they overlap its Riemann term instead of stalling the lane
       struct Cand {
         R2 p, v, r;
-        int fl, l;
+        int fl;
       };
-      auto eval2 = [&](unsigned ma, int sa0, unsigned mb, int sb0) {
+      // M32 forms r^2 and q of the last candidate with the products in the other order (swap), as
+      // the fused loop has always rounded them; not when the lane itself, which is left out, came last
+      auto eval2 = [&](unsigned ma, int sa0, unsigned mb, int sb0, bool self_last) {
         unsigned long long m = (unsigned long long)ma | ((unsigned long long)mb << 32);
         if (m == 0ull) return;
         const int sb = sb0 - 32;
@@ -1823,11 +1868,11 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
           const int b = __builtin_ctzll(m);
           m &= m - 1ull;
           const int l = (b < 32 ? sa0 : sb) + b;
-          return Cand{s_pos[l], s_vel[l], s_rp[l], (int)s_fl[l], l};
+          return Cand{s_pos[l], s_vel[l], s_rp[l], (int)s_fl[l]};
         };
-        auto use = [&](const Cand &q) {
+        auto use = [&](const Cand &q, bool swap) {
           const R dx = q.p.x - xi, dy = q.p.y - yg;
-          fluid_j(Inside{}, false, dx, dy, norm2(dx, dy), q.v.x, q.v.y, q.r.x, q.r.y, q.fl, true);
+          fluid_j(Inside{}, false, swap, dx, dy, q.v.x, q.v.y, q.r.x, q.r.y, q.fl, true);
         };
         Cand cur = next();
         // unrolled by two, so that every other round reads into the registers the previous one
@@ -1835,18 +1880,19 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
 #pragma unroll 2
         while (m) {
           const Cand nxt = next();
-          use(cur);
+          use(cur, false);
           cur = nxt;
         }
-        use(cur);
+        use(cur, !self_last);
       };
-      auto eval = [&](unsigned m, int s0) { eval2(m, s0, 0u, 0); };
+      auto eval = [&](unsigned m, int s0, bool self_last) { eval2(m, s0, 0u, 0, self_last); };
       const int off = lsx - P.sc0;  // tile sub-column of the lane's own sub-column
       // the windows are marked left to right (offsets -3 .. +3; window q has offset
       // window_offset(q)), the order in which a recording keeps its runs for the shift passes;
       // a recording widens them by the skin
       const float Rpw = record ? Rp + cp.skin_grow : Rp;
-      unsigned dmask = 0u;  // windows evaluated whole
+      bool own_last = false;  // the lane itself was its window's last marked candidate
+      unsigned dmask = 0u;    // windows evaluated whole
 #pragma unroll
       for (int k = 0; k < kWindowOrder; ++k) {
         const int o = k - 3, q = o < 0 ? -2 * o - 1 : 2 * o;
@@ -1875,7 +1921,10 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
         }
         // the lane itself (in the window of its own sub-column): no term, and no FREE_SURFACE
         // neighbour of its own
-        if (o == 0 && own >= s0 && own < s1) mk[q] &= ~(1u << (own - s0));
+        if (o == 0 && own >= s0 && own < s1) {
+          own_last = (mk[q] >> (own - s0)) == 1u;
+          mk[q] &= ~(1u << (own - s0));
+        }
       }
       if (record) d.f_wc[i] = rr.entry(cum0);
       // windows in the order 0, -1, +1, ... (those at -k and +k in one loop unless one of them
@@ -1884,7 +1933,7 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
         if ((dmask >> q) & 1u)
           direct(w0[q], (int)mk[q]);
         else
-          eval(mk[q], w0[q]);
+          eval(mk[q], w0[q], q == 0 && own_last);
       };
       evalq(0);
 #pragma unroll
@@ -1893,7 +1942,7 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
           evalq(q);
           evalq(q + 1);
         } else {
-          eval2(mk[q], w0[q], mk[q + 1], w0[q + 1]);
+          eval2(mk[q], w0[q], mk[q + 1], w0[q + 1], false);
         }
       }
       if (wstaged) {  // walls of the 3x3 cells, cell column by cell column
@@ -1905,7 +1954,7 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
             direct(s0, s1);
           } else {
             unsigned ms;
-            eval(mark(std::false_type{}, s0, s1, ms), s0);
+            eval(mark(std::false_type{}, s0, s1, ms), s0, false);
           }
         }
       }
@@ -1934,10 +1983,10 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
           const R dx = ld32(d.w_vx, s) - bx, dy = ld32(d.w_vy, s) - by;
           const R r2 = norm2(dx, dy);
           if (!(r2 < K.rc2)) return;
-          const R w = K.gauss_in(r2);
+          const R w = K.w_in(r2);
           const int phj = d.w_phase[s];
-          riemann_pair<R, VISCID>(dx, dy, r2, w, ui, vi, d.w_u[s], d.w_v[s], rhoi, cp.rho0[phj], pi, d.w_p[s], cs,
-                                  csinv, hmu, eps_h2, S);
+          const R du_ = ui - d.w_u[s], dv_ = vi - d.w_v[s];
+          riemann_pair<R, VISCID, true>(dx, dy, r2, kfma(du_, dx, dv_ * dy), w, du_, dv_, cp.rho0[phj], d.w_p[s], I, S);
           S.col = kfma(r2, phj == col_skip ? R(0) : w, S.col);
         });
       }
@@ -1956,13 +2005,13 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
           const R dx = d.s_vx[j] - bx, dy = d.s_vy[j] - by;
           const R r2 = norm2(dx, dy);
           if (!(r2 < K.rc2)) return;
-          const R w = K.gauss_in(r2);
-          riemann_pair<R, VISCID>(dx, dy, r2, w, ui, vi, (R)d.su[j], (R)d.sv[j], rhoi, rhoi, pi, d.s_p[j], cs, csinv,
-                                  hmu, eps_h2, S);
+          const R w = K.w_in(r2);
+          const R du_ = ui - (R)d.su[j], dv_ = vi - (R)d.sv[j];
+          riemann_pair<R, VISCID>(dx, dy, r2, kfma(du_, dx, dv_ * dy), w, du_, dv_, rhoi, d.s_p[j], I, S);
         });
       }
     }
-    pair_finish(S, rhoi, K.kdc);
+    pair_finish(S, I);
     d.f_col[i] = S.col;
     const int near = !liq ? 0 : S.fsr < qrc2 ? 2 : (S.fsr < K.rc2 ? 1 : 0);
     d.f_near[i] = (int8_t)near;
@@ -2126,8 +2175,8 @@ __device__ __forceinline__ void shift_tile(const Dev<Pol> &d, const TilePlan &P,
     lp = lane_pos(x0, y0, lsx, sy, cp);
   const LoopConsts<R> K(cp);
   R gx = 0, gy = 0;
-  auto add = [&](R dx, R dy) {  // (kd c32 multiplies the sums, below)
-    const R w = K.gauss(norm2(dx, dy));
+  auto add = [&](R dx, R dy) {  // (P64: kd c32 multiplies the sums, below)
+    const R r2 = norm2(dx, dy), w = Pol::MIXED ? K.w(r2) : K.gauss(r2);
     gx = kfma(dx, w, gx);
     gy = kfma(dy, w, gy);
   };
@@ -2263,11 +2312,12 @@ __device__ __forceinline__ void shift_tile(const Dev<Pol> &d, const TilePlan &P,
       });
     }
   }
-  gx *= K.kdc;
-  gy *= K.kdc;
   if constexpr (Pol::MIXED) {
     gx = kfma(gxs, cp.kdc_s, gx);
     gy = kfma(gys, cp.kdc_s, gy);
+  } else {
+    gx *= K.kdc;
+    gy *= K.kdc;
   }
   const R umax = d.umax[c];
   const R shift_k = (R)(cp.shift_ch * d.dtv[c]);  // particle_shift_coef h dt
@@ -2291,25 +2341,26 @@ __device__ __forceinline__ void shift_tile(const Dev<Pol> &d, const TilePlan &P,
     sxv = kfma(kfma(-nx, nx, R(1)), dxs, -((nx * ny) * dys));
     syv = kfma(kfma(-ny, ny, R(1)), dys, -((ny * nx) * dxs));
   }
-  sxv *= umax;
-  syv *= umax;
-  const R2 sn{sacc.x + sxv, sacc.y + syv};
+  // the speed factor comes in with the sums it is added to, fused
+  const R2 sn{kfma(sxv, umax, sacc.x), kfma(syv, umax, sacc.y)};
   double x = 0.0, y = 0.0;
   if constexpr (Pol::MIXED) {
     // the views move by this pass's shift in float; the masters take the accumulated shift
     // in double on the last pass
-    B.vx[i] = xi + sxv;
-    B.vy[i] = yi + syv;
+    B.vx[i] = kfma(sxv, umax, xi);
+    B.vy[i] = kfma(syv, umax, yi);
     if (last) {
       x = x0 + (double)sn.x;
       y = y0 + (double)sn.y;
     }
   } else {
-    x = x0 + sxv;
-    y = y0 + syv;
+    x = kfma(sxv, umax, x0);
+    y = kfma(syv, umax, y0);
     B.x[i] = x;
     B.y[i] = y;
   }
+  sxv *= umax;
+  syv *= umax;
   // path length: this pass moved the particle by (sxv, syv); the passes after a recording
   // one count from it and the last adds the path since the hash it recorded
   const float sx2 = (float)sxv, sy2 = (float)syv, step = __builtin_amdgcn_sqrtf(norm2(sx2, sy2));
@@ -2480,7 +2531,7 @@ __device__ __forceinline__ void solid_couple_block(const Dev<Pol> &d, int bid) {
     const int pk = d.s_cxy[i], cx = cxy_x(pk), cy = cxy_y(pk);
     const R xi = d.s_vx[i], yi = d.s_vy[i];
     const LoopConsts<R> K(cp);
-    const R eR = cp.eR, k2c = cp.k2c, nhl2 = cp.nhl2;
+    const R eR = cp.eR, k2c = cp.k2c, hinv2 = cp.hinv2, nhl2 = cp.nhl2;
     const auto &F = d.fa;
     // fluid: the 3x3 cells' 18 runs spread over the group's lanes (as in the force kernel)
     for (int r = l; r < kCellRuns; r += kSolidLanes) {
@@ -2491,7 +2542,7 @@ __device__ __forceinline__ void solid_couple_block(const Dev<Pol> &d, int bid) {
         const R dx = f.x - bx, dy = f.y - by;
         const R r2 = dx * dx + dy * dy;
         if (r2 < K.rc2) {
-          const R w = (kgauss<R>(r2, nhl2) - eR) * k2c;
+          const R w = (kgauss2<R>(r2, hinv2, nhl2) - eR) * k2c;
           S += w;
           P += f.p * w;
         }

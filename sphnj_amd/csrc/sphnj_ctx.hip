@@ -252,6 +252,7 @@ struct Engine : EngineBase {
     std::memset(&c, 0, sizeof(c));
     c.rc2 = (R)D.rc2;
     c.quarter_rc2 = (R)(0.25 * D.rc2);
+    c.hinv2 = (R)D.hinv2;
     c.nhl2 = (R)(-D.hinv2 * 1.4426950408889634);
     c.kdc = (R)D.kdc;
     {
