@@ -1820,36 +1820,35 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
       };
       auto mark = [&](auto rec, int s0, int s1, unsigned &ms) -> unsigned {
         constexpr bool REC = decltype(rec)::value;
-        ms = 0u;
-        // 4 candidates a round (then 2, then 1), their bits gathered in a nibble placed at
-        // once, so that the bit positions cost no instruction per candidate
+        // whole rounds of 4 candidates (up to 3 past the run: the next span's or padding, dropped
+        // below); a test's carry goes in with the doubling of the mask, one instruction, so the
+        // first candidate ends up highest and the masks are reversed at the end.  With the bits
+        // gathered by selects and a tail of 2 and 1 candidates a round took 42 instead of 36
+        // instructions (31 to 27 without the recording)
         auto r2of = [&](const R2 &pj) {
           const R dx = pj.x - xi, dy = pj.y - yg;
           return norm2(dx, dy);
         };
         const R rc2 = K.rc2;
-        unsigned m = 0u;
-        int s = s0, sh = 0;
+        unsigned m = 0u, w = 0u;
 #pragma unroll 1
-        for (const int last = s1 - 3; s < last; s += 4, sh += 4) {
+        for (int s = s0; s < s1; s += 4) {
           const R2 p0 = s_pos[s], p1 = s_pos[s + 1], p2 = s_pos[s + 2], p3 = s_pos[s + 3];
           const R q0 = r2of(p0), q1 = r2of(p1), q2 = r2of(p2), q3 = r2of(p3);
-          m |= ((q0 < rc2 ? 1u : 0u) | (q1 < rc2 ? 2u : 0u) | (q2 < rc2 ? 4u : 0u) | (q3 < rc2 ? 8u : 0u)) << sh;
-          if (REC) ms |= ((q0 < rl2 ? 1u : 0u) | (q1 < rl2 ? 2u : 0u) | (q2 < rl2 ? 4u : 0u) | (q3 < rl2 ? 8u : 0u)) << sh;
+          m = m + m + (q0 < rc2 ? 1u : 0u);
+          m = m + m + (q1 < rc2 ? 1u : 0u);
+          m = m + m + (q2 < rc2 ? 1u : 0u);
+          m = m + m + (q3 < rc2 ? 1u : 0u);
+          if (REC) {
+            w = w + w + (q0 < rl2 ? 1u : 0u);
+            w = w + w + (q1 < rl2 ? 1u : 0u);
+            w = w + w + (q2 < rl2 ? 1u : 0u);
+            w = w + w + (q3 < rl2 ? 1u : 0u);
+          }
         }
-        if (s + 1 < s1) {
-          const R q0 = r2of(s_pos[s]), q1 = r2of(s_pos[s + 1]);
-          m |= ((q0 < rc2 ? 1u : 0u) | (q1 < rc2 ? 2u : 0u)) << sh;
-          if (REC) ms |= ((q0 < rl2 ? 1u : 0u) | (q1 < rl2 ? 2u : 0u)) << sh;
-          s += 2;
-          sh += 2;
-        }
-        if (s < s1) {
-          const R q0 = r2of(s_pos[s]);
-          m |= (q0 < rc2 ? 1u : 0u) << sh;
-          if (REC) ms |= (q0 < rl2 ? 1u : 0u) << sh;
-        }
-        return m;
+        const int n = s1 - s0, drop = -n & 3, up = -n & 31;
+        ms = REC ? __builtin_bitreverse32((w >> drop) << up) : 0u;
+        return __builtin_bitreverse32((m >> drop) << up);
       };
       // the marked candidates of window (ma, sa0) and then of window (mb, sb0), in slot order;
       // the LDS reads of the next candidate are issued before the current one is summed, so
@@ -1859,8 +1858,9 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
         int fl;
       };
       // M32 forms r^2 and q of the last candidate with the products in the other order (swap), as
-      // the fused loop has always rounded them; not when the lane itself, which is left out, came last
-      auto eval2 = [&](unsigned ma, int sa0, unsigned mb, int sb0, bool self_last) {
+      // the fused loop has always rounded them; not with no_swap (the lane itself, which is left
+      // out, came last)
+      auto eval2 = [&](unsigned ma, int sa0, unsigned mb, int sb0, bool no_swap) {
         unsigned long long m = (unsigned long long)ma | ((unsigned long long)mb << 32);
         if (m == 0ull) return;
         const int sb = sb0 - 32;
@@ -1883,9 +1883,8 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
           use(cur, false);
           cur = nxt;
         }
-        use(cur, !self_last);
+        use(cur, !no_swap);
       };
-      auto eval = [&](unsigned m, int s0, bool self_last) { eval2(m, s0, 0u, 0, self_last); };
       const int off = lsx - P.sc0;  // tile sub-column of the lane's own sub-column
       // the windows are marked left to right (offsets -3 .. +3; window q has offset
       // window_offset(q)), the order in which a recording keeps its runs for the shift passes;
@@ -1903,8 +1902,7 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
         if (!span_window(P, cp, lsx, sa, sy, cy, lp, Rpw, ra, rb)) continue;
         const int s0 = s_lb[sa][ra - P.r0], s1 = s_lb[sa][rb + 1 - P.r0];
         w0[q] = s0;
-        if (s1 - s0 > 32) {  // evaluated whole below; its end in place of the mask
-          mk[q] = (unsigned)s1;
+        if (s1 - s0 > 32) {  // evaluated whole below
           dmask |= 1u << q;
           rr.ok = false;
           continue;
@@ -1927,34 +1925,60 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
         }
       }
       if (record) d.f_wc[i] = rr.entry(cum0);
-      // windows in the order 0, -1, +1, ... (those at -k and +k in one loop unless one of them
-      // is evaluated whole)
-      auto evalq = [&](int q) {
-        if ((dmask >> q) & 1u)
-          direct(w0[q], (int)mk[q]);
-        else
-          eval(mk[q], w0[q], q == 0 && own_last);
-      };
-      evalq(0);
+      // windows in the order 0, -1, +1, ..., those at -k and +k in one loop
+      if (dmask == 0u) {
+        eval2(mk[0], w0[0], 0u, 0, own_last);
 #pragma unroll
-      for (int q = 1; q < kWindowOrder; q += 2) {
-        if (((dmask >> q) & 3u) != 0u) {
-          evalq(q);
-          evalq(q + 1);
-        } else {
-          eval2(mk[q], w0[q], mk[q + 1], w0[q + 1], false);
+        for (int q = 1; q < kWindowOrder; q += 2) eval2(mk[q], w0[q], mk[q + 1], w0[q + 1], false);
+      } else {  // a lane with a window evaluated whole (rare): the windows once more, one loop of code
+#pragma unroll 1
+        for (int k = 0; k < 4; ++k) {
+          const int q = k == 0 ? 0 : 2 * k - 1;  // window 0, then the pairs 1 2, 3 4, 5 6
+          int s0[2] = {0, 0}, s1[2] = {0, 0};
+          bool whole = false;
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const int sa = off + window_offset(q + h);
+            int ra, rb;
+            if ((h == 1 && k == 0) || !span_window(P, cp, lsx, sa, sy, cy, lp, Rpw, ra, rb)) continue;
+            s0[h] = s_lb[sa][ra - P.r0];
+            s1[h] = s_lb[sa][rb + 1 - P.r0];
+            whole = whole || s1[h] - s0[h] > 32;
+          }
+          unsigned m[2], ms;
+#pragma unroll
+          for (int h = 0; h < 2; ++h) m[h] = s1[h] - s0[h] > 32 ? 0u : mark(std::false_type{}, s0[h], s1[h], ms);
+          bool last0 = false;
+          if (k == 0 && m[0] != 0u && own >= s0[0] && own < s1[0]) {
+            last0 = (m[0] >> (own - s0[0])) == 1u;
+            m[0] &= ~(1u << (own - s0[0]));
+          }
+          if (whole) {
+#pragma unroll 1
+            for (int h = 0; h < 2; ++h) {
+              const int a = h ? s0[1] : s0[0], b = h ? s1[1] : s1[0];
+              if (b - a > 32)
+                direct(a, b);
+              else
+                eval2(h ? m[1] : m[0], a, 0u, 0, false);
+            }
+          } else {
+            eval2(m[0], s0[0], m[1], s0[1], last0);
+          }
         }
       }
-      if (wstaged) {  // walls of the 3x3 cells, cell column by cell column
+      if (wstaged) {
+        // walls of the 3x3 cells, cell column by cell column, at most 32 marked at a time (a
+        // column beside a side wall holds about 47, of which some 20 lie inside the cut-off;
+        // evaluated whole they made the walls' waves the slowest of a launch)
         const int lr0 = max(cy - 1, 0) - W.wcr0, lr1 = min(cy + 1, cp.ny - 1) - W.wcr0;
-#pragma unroll
+#pragma unroll 1
         for (int a = 0; a < 3; ++a) {
           const int s0 = s_wlb[a][lr0], s1 = s_wlb[a][lr1 + 1];
-          if (s1 - s0 > 32) {
-            direct(s0, s1);
-          } else {
+#pragma unroll 1
+          for (int b = s0; b < s1; b += 32) {
             unsigned ms;
-            eval(mark(std::false_type{}, s0, s1, ms), s0, false);
+            eval2(mark(std::false_type{}, b, min(b + 32, s1), ms), b, 0u, 0, s1 - s0 > 32);
           }
         }
       }
