@@ -121,6 +121,10 @@ struct Dev {
   // staged candidates
   uint4 *f_wc;
   float *tile_d0;
+  // per global cell column (ncol of them), two sets by shift-pass parity: non-zero where a lane's
+  // path since the runs' recording exceeds half the skin
+  int *f_far;
+  int ncol;
   int2 *f_srange;  // per global sub-cell (4 per cell): [start, end) slot range, empty (0, 0)
   // per sub-column, 2 ny + 1 entries: first slot of sub-row k or later; the sub-column's end
   int *f_lb;

@@ -406,6 +406,7 @@ __global__ void __launch_bounds__(256) k_permute_fluid(Dev<Pol> d) {
     d.umax2[i] = 0ull;
     d.umax[i] = 0;
   }
+  for (int k = i; k < 2 * d.ncol; k += gridDim.x * blockDim.x) d.f_far[k] = 0;
   if (i >= d.nf) return;
   // counting sort, step 5: inside each key, slots in original-index order -- a slot's place is
   // its key's start plus the number of the key's slots with a smaller original index -- so the
@@ -750,10 +751,10 @@ struct V2<double> {
   using T = double2;
 };
 
-struct TilePlan {
+struct alignas(16) TilePlan {  // (read by scalar loads)
   int c, start, count;   // case, slot of lane 0, lanes
   int start1, count0;    // lanes [count0, count) are the slots from start1 on (odd sub-column)
-  int sx, cx;            // even sub-column and cell column of the tile
+  int sx, cx, gcol;      // even sub-column and cell column of the tile; global cell column
   int sc0, nsc, r0, nr;  // candidate sub-columns and sub-rows
   int cy_ref;            // cell row of the M32 shift frame
   int sw;                // wall (bit 0) / solid (bit 1) particles lie in the tile's 3x3 cells
@@ -1113,6 +1114,7 @@ __global__ void __launch_bounds__(256) k_tile_plan(Dev<Pol> d, int G, const int 
     P.count0 = count0;
     P.sx = sx;
     P.cx = cx;
+    P.gcol = g >> 1;
     P.sc0 = sc0;
     P.nsc = nsc;
     P.r0 = r0;
@@ -1196,19 +1198,19 @@ __global__ void __launch_bounds__(64) k_umax_final(Dev<Pol> d) {
   }
 }
 
-// Copies a tile into LDS: the row tables (lb[a][k] = LDS index of the first candidate of row
-// r0 + k or later of sub-column sc0 + a, k = 0..nr) and, through ld / st, the candidates:
-// span a occupies LDS [base[a], base[a] + len[a]) in slot order.  Each span is served by a
-// contiguous group of threads (its rows and its particles, coalesced), so every element's
-// span is known without a search; the loads of U particles are issued before any is
-// stored.  st(l, v, a) receives the span too.
-template <int BLOCK, int U, class Ld, class St>
+// Copies a tile into LDS: the row tables (lb[a][k] = LDS index of the first candidate
+// of row r0 + k or later of sub-column sc0 + a, k = 0..nr) and, through ld / st, the candidates:
+// span a occupies LDS [base[a], base[a] + len[a]) in slot order, PAD free entries after it.  Each
+// span is served by a contiguous group of threads (its rows and its particles, coalesced), so
+// every element's span is known without a search; the loads of U particles are issued before any
+// is stored.  st(l, v, a) receives the span too.
+template <int BLOCK, int U, int PAD, class Ld, class St>
 __device__ __forceinline__ void tile_stage(const TilePlan &P, const int *f_lb, int (*lb)[TileRows<BLOCK>::value + 1],
                                            Ld &&ld, St &&st) {
   const int t = threadIdx.x, n = P.nsc, nr = P.nr, gsz = P.gsz;
   const int a = min((int)(((unsigned)t * (unsigned)P.gmul) >> 20), n - 1), k0 = t - a * gsz;
   const int stride = a == n - 1 ? BLOCK - a * gsz : gsz;
-  int base = 0;
+  int base = PAD * a;
   for (int q = 0; q < a; ++q) base += P.len[q];
   const int lo = P.lo[a], len = P.len[a], row = P.row[a];
   for (int k = k0; k <= nr; k += stride) lb[a][k] = f_lb[row + k] - lo + base;
@@ -1332,22 +1334,34 @@ __device__ __forceinline__ bool span_window(const TilePlan &P, const CP &cp, int
 }
 
 // Shift windows over the passes of a step.  A step's shift passes move particles by a tiny
-// fraction of rc, and every pass of a step uses the same tiles, so the same staged LDS
-// order.  The first pass (kShiftRecord, when a step has more than one) widens its pruning
-// radius by s rc and records, per lane and candidate sub-column, the run of LDS indices from
-// the first to the last candidate within rc (1 + s).  Its path lengths restart: the lanes
-// store the path since that pass (and keep the one since the hash with the runs).  A later
-// pass (kShiftCached) walks only those runs while the lane's path since the first pass plus
-// the largest one among the tile's staged candidates stays within s rc: every candidate
-// within rc then was within rc (1 + s) at the first pass, so it lies in a run, and the runs
-// keep the sub-column and slot order, so the non-zero terms and their order are those of the
-// full windows and the sums are the same bit for bit.  Any other lane searches the full
-// windows, with the tile's path bound rebuilt from the first pass's bound.  The last pass
-// writes the path since the hash again.  kShiftPlain is the single pass of a one-pass step.
-// When the pair kernel runs on the shift's tiles it records the runs itself, at the hash's
-// positions (with the lane's path since the hash and the tile's staged path bound, as the
+// fraction of rc, and every pass of a step uses the same tiles.  The first pass (kShiftRecord,
+// when a step has more than one) widens its pruning radius by s rc and records, per lane and
+// candidate sub-column, the run of LDS indices from the first to the last candidate within
+// rc (1 + s), in the layout in which a kShiftCached pass stages the tile (every span followed by
+// kRunPad far-away entries).  Its path lengths restart: the lanes store the path since that pass
+// (and keep the one since the hash with the runs).  A later pass (kShiftCached) walks only those
+// runs while the lane's path since the first pass plus the largest one among its candidates stays
+// within s rc: every candidate within rc then was within rc (1 + s) at the first pass, so it
+// lies in a run, and the runs keep the sub-column and slot order, so the non-zero terms and their
+// order are those of the full windows and the sums are the same bit for bit.  Any other lane
+// searches the full windows, with the tile's path bound rebuilt from the first pass's bound.
+//   What bounds the candidates' paths is a flag per cell column (f_far): a pass, and the pair
+// kernel before the first, raises its column's where a lane's path exceeds half of s rc.  With
+// none raised in a tile's three columns every two paths together are within s rc and nothing of
+// the candidates but their positions is staged; with one raised the tile stages their paths'
+// maximum and each lane is tested.  A pass reads the flags the launch before it wrote and writes
+// the other set (two sets by pass parity), so none changes while it is read; a path only grows, so
+// a set that is not cleared between its uses only says too much.
+//   The last pass writes the path since the hash again.  kShiftPlain is the single pass of a
+// one-pass step.  When the pair kernel runs on the shift's tiles it records the runs itself, at the
+// hash's positions (with the lane's path since the hash and the tile's staged path bound, as the
 // first pass would), and every pass of the step is a kShiftCached one: the paths then count
 // from the hash, which bounds the paths since the recording.
+//   A run is walked in whole groups of kRunPad + 1 (M32 4, P64 2: its four candidates' FP64 terms
+// in flight cost more registers than they hide): entries past its end lie beyond rc (its span's
+// next candidates) or far away (the padding), and add exact zeros.
+template <class Pol>
+constexpr int kRunPad = Pol::MIXED ? 3 : 1;
 constexpr int kShiftPlain = 0, kShiftRecord = 1, kShiftCached = 2;
 constexpr double kShiftSkin = 0.02;
 
@@ -1664,7 +1678,7 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
     const auto &cq = d.cases[c];
     const R fdx = cq.cdx_r, fdy = cq.cdy_r;
     const int gcx = P.cx, gcy = P.cy_ref;
-    tile_stage<BLOCK, 4>(
+    tile_stage<BLOCK, 4, 0>(
         P, d.f_lb, s_lb,
         [&](int g) {
           return Ld{R2{ld32(A.vx, g), ld32(A.vy, g)}, R2{ld32(A.vu, g), ld32(A.vv, g)},
@@ -1912,7 +1926,7 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
           mk[q] = mark(std::true_type{}, s0, s1, ms);
           if (ms != 0u) {
             const int f = __builtin_ctz(ms);
-            rr.put(s0 + f, 32 - __builtin_clz(ms) - f);
+            rr.put(s0 + kRunPad<Pol> * sa + f, 32 - __builtin_clz(ms) - f);
           }
         } else {
           mk[q] = mark(std::false_type{}, s0, s1, ms);
@@ -2088,7 +2102,9 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
     const double u2 = norm2(u, v);
     my_u2 = (unsigned long long)__double_as_longlong(u2);
     const double mx = x - x0, my = y - y0;
-    B.cum[i] = (float)((double)cum0 + sqrt(norm2(mx, my)));
+    const float path = (float)((double)cum0 + sqrt(norm2(mx, my)));
+    B.cum[i] = path;
+    if (path > 0.5f * cp.skin_ok) d.f_far[P.gcol] = 1;  // read by the first shift pass
     if (isnan(rho) || isnan(x) || isnan(y) || isnan(u2)) atomicOr(d.status, kStNaN);
   }
   // per-case max |u|^2 (non-negative doubles order like their bit patterns)
@@ -2160,10 +2176,10 @@ __device__ __forceinline__ ShiftOwn<Pol> shift_own(const Dev<Pol> &d, const Tile
 // Reads only the LDS it is given; stores only the lanes' own results.  D bounds the staged
 // candidates' paths since the hash; a cached pass also passes Dsp, their paths since the
 // step's first pass, and runs whether a staged tile may walk the recorded runs.
-template <class Pol, int BLOCK, int MODE, class LB, int WROWS>
+template <class Pol, int BLOCK, int MODE, int WROWS>
 __device__ __forceinline__ void shift_tile(const Dev<Pol> &d, const TilePlan &P, int pass, const ShiftOwn<Pol> &own,
                                            const typename V2<typename Pol::R>::T *s_pos,
-                                           const LB (*s_lb)[TileRows<BLOCK>::value + 1], const int (*s_wlb)[WROWS + 1],
+                                           const int (*s_lb)[TileRows<BLOCK>::value + 1], const int (*s_wlb)[WROWS + 1],
                                            float D, float Dsp, bool runs, bool staged, bool wstaged,
                                            const WallSpans &W) {
 #pragma clang fp contract(off)
@@ -2211,10 +2227,14 @@ __device__ __forceinline__ void shift_tile(const Dev<Pol> &d, const TilePlan &P,
   // rescaled below), the lane's own entry giving its position there
   R gxs = 0, gys = 0;
   R xs = xi, ys = yi;
+  constexpr int PAD = MODE == kShiftCached ? kRunPad<Pol> : 0;
+  auto span_base = [&](int sa) {  // LDS index of the first candidate of span sa
+    int b = PAD * sa;
+    for (int a = 0; a < sa; ++a) b += P.len[a];
+    return b;
+  };
   if (staged) {
-    int own = i - P.lo[lsx - P.sc0];
-    for (int a = 0; a < lsx - P.sc0; ++a) own += P.len[a];
-    const R2 o = s_pos[own];
+    const R2 o = s_pos[i - P.lo[lsx - P.sc0] + span_base(lsx - P.sc0)];
     xs = o.x;
     ys = o.y;
   }
@@ -2242,11 +2262,18 @@ __device__ __forceinline__ void shift_tile(const Dev<Pol> &d, const TilePlan &P,
   if (cached) {
     const unsigned x = own.wc.x, y = own.wc.y, z = own.wc.z;
     const int s0 = x & 0x7ff, s1 = (x >> 11) & 0x7ff, s2 = y & 0x7ff, s3 = (y >> 11) & 0x7ff, s4 = z & 0x7ff;
-    for_range_4_2_1(s0, s0 + (int)((x >> 22) & 0x7f), staged_add);
-    for_range_4_2_1(s1, s1 + (int)((y >> 22) & 0x7f), staged_add);
-    for_range_4_2_1(s2, s2 + (int)((z >> 11) & 0x7f), staged_add);
-    for_range_4_2_1(s3, s3 + (int)((z >> 18) & 0x7f), staged_add);
-    for_range_4_2_1(s4, s4 + (int)(z >> 25), staged_add);
+    auto walk = [&](int lo, int n) {
+#pragma unroll 1
+      for (int l = lo, hi = lo + n; l < hi; l += kRunPad<Pol> + 1) {
+#pragma unroll
+        for (int k = 0; k <= kRunPad<Pol>; ++k) (void)staged_term(l + k);
+      }
+    };
+    walk(s0, (int)((x >> 22) & 0x7f));
+    walk(s1, (int)((y >> 22) & 0x7f));
+    walk(s2, (int)((z >> 11) & 0x7f));
+    walk(s3, (int)((z >> 18) & 0x7f));
+    walk(s4, (int)(z >> 25));
   } else {
     const R rl2 = cp.rl2_rec;
     for_windows<false>(P, cp, lsx, sy, cy, lp, Rp, [&](int sc, int ra, int rb) {
@@ -2276,7 +2303,7 @@ __device__ __forceinline__ void shift_tile(const Dev<Pol> &d, const TilePlan &P,
             if (l < hi) mk |= (staged_term(l) < rl2 ? 1u : 0u) << sh;
             if (mk != 0u) {
               const int f = __builtin_ctz(mk);
-              rr.put(lo + f, 32 - __builtin_clz(mk) - f);
+              rr.put(lo + kRunPad<Pol> * sa + f, 32 - __builtin_clz(mk) - f);
             }
           } else {  // f follows l until one is seen
             int f = lo, la = lo;
@@ -2287,7 +2314,7 @@ __device__ __forceinline__ void shift_tile(const Dev<Pol> &d, const TilePlan &P,
               seen = seen || in;
               la = in ? q : la;
             });
-            if (seen) rr.put(f, la - f + 1);
+            if (seen) rr.put(f + kRunPad<Pol> * sa, la - f + 1);
           }
         } else {
           for_range_4_2_1(lo, hi, staged_add);
@@ -2388,12 +2415,13 @@ __device__ __forceinline__ void shift_tile(const Dev<Pol> &d, const TilePlan &P,
   // path length: this pass moved the particle by (sxv, syv); the passes after a recording
   // one count from it and the last adds the path since the hash it recorded
   const float sx2 = (float)sxv, sy2 = (float)syv, step = __builtin_amdgcn_sqrtf(norm2(sx2, sy2));
-  if constexpr (MODE == kShiftPlain)
+  if constexpr (MODE == kShiftPlain) {
     B.cum[i] = cum0 + step;
-  else if constexpr (MODE == kShiftRecord)
-    B.cum[i] = last ? cum0 + step : step;
-  else
-    B.cum[i] = last ? (own.cum_hash + cum0) + step : cum0 + step;
+  } else {
+    const float path = MODE == kShiftRecord ? step : cum0 + step;  // since the recording
+    if (path > 0.5f * cp.skin_ok) d.f_far[((pass + 1) & 1) * d.ncol + P.gcol] = 1;
+    B.cum[i] = last ? (MODE == kShiftRecord ? cum0 + step : (own.cum_hash + cum0) + step) : path;
+  }
   if (last) {
     if constexpr (Pol::MIXED) {
       A.x[i] = x;
@@ -2412,10 +2440,13 @@ __device__ __forceinline__ void shift_tile(const Dev<Pol> &d, const TilePlan &P,
 // correctionCalculate (src/fluid.cu:316-367) + correctionUpdate / shiftDisplacementCalculate
 // (src/fluid.cu:369-427), one tile per block: stage the tile, then shift_tile.  MODE is
 // kShiftPlain, kShiftRecord or kShiftCached (the step's one pass, its first of several, a
-// later one).  The cached passes are held to 8 waves per SIMD (64 registers, a few spilled:
-// 6% faster than 7), the others to 7.
+// later one).  Held to 7 waves per SIMD: vector issue bounds the M32 passes (0.95 instructions a
+// CU-cycle on the 3.0 M dam break, 92 us a pass), and an eighth wave costs spills (95 us).  Without
+// the candidates' paths in the staging and with whole groups in the runs a pass of the 187 k
+// two-phase case takes 18.3 us instead of 19.2, of the 5 k dam break 10.8 instead of 11.3, of the
+// 3.0 M case what it took (its runs' 88 slots per wave, for 45 neighbours a lane, are the rest).
 template <class Pol, int BLOCK, int MODE>
-__global__ void __launch_bounds__(BLOCK, (MODE == kShiftCached ? 8 : 7))
+__global__ void __launch_bounds__(BLOCK, 7)
     k_fluid_shift(Dev<Pol> d, const TilePlan *plans, const int *ntiles, int pass, int use_runs) {
   using R = typename Pol::R;
   using R2 = typename V2<R>::T;
@@ -2423,8 +2454,10 @@ __global__ void __launch_bounds__(BLOCK, (MODE == kShiftCached ? 8 : 7))
   // walls of the tile's 3x3 cell columns over its cell rows follow the fluid candidates
   // (a tile's fluid candidates rarely fill CAP, so the walls also use what they leave)
   constexpr int WCAP = BLOCK / 2, WROWS = TileRows<BLOCK>::value / 2 + 2;
-  // fluid candidates, padding, walls, padding (the padding is far away: read by masked tails)
-  __shared__ R2 s_pos[CAP + WCAP + 8];
+  constexpr bool CACHED = MODE == kShiftCached;
+  constexpr int PAD = CACHED ? kRunPad<Pol> : 0, PADS = PAD * kTileCols;
+  // fluid candidates, padding, walls, padding (the padding is far away: read past a run's end)
+  __shared__ R2 s_pos[CAP + PADS + WCAP + 8];
   __shared__ int s_lb[kTileCols][TileRows<BLOCK>::value + 1];
   __shared__ int s_wlb[3][WROWS + 1];  // LDS index of the first wall of cell row wcr0 + k or later
   __shared__ float s_dmax[BLOCK / 64];
@@ -2437,6 +2470,13 @@ __global__ void __launch_bounds__(BLOCK, (MODE == kShiftCached ? 8 : 7))
   const bool staged = P.total <= CAP && P.nr <= TileRows<BLOCK>::value;
   const ShiftOwn<Pol> own = shift_own<Pol, MODE>(d, P, pass, cp.K);
   int dmax = 0;  // bit pattern of the largest path length (non-negative floats order as ints)
+  // a cached pass: whether some path in the tile's columns exceeds half the skin
+  int far = 0;
+  if constexpr (CACHED) {
+    const int *ff = d.f_far + (pass & 1) * d.ncol + (P.gcol - P.cx);
+    far = ff[P.sc0 >> 1] | ff[P.cx] | ff[(P.sc0 + P.nsc - 1) >> 1];
+  }
+  const int total = P.total + PAD * P.nsc;  // staged entries of the fluid
   if (staged) {
     struct Ld {
       R2 pos;
@@ -2448,24 +2488,36 @@ __global__ void __launch_bounds__(BLOCK, (MODE == kShiftCached ? 8 : 7))
     const int sa = min((int)(((unsigned)t * (unsigned)P.gmul) >> 20), P.nsc - 1);
     const R xo = (R)(((P.sc0 + sa) >> 1) - P.cx) * cp.cdx_r * gs;
     const int gcy = P.cy_ref;
-    tile_stage<BLOCK, 4>(
+    tile_stage<BLOCK, 4, PAD>(
         P, d.f_lb, s_lb,
         [&](int g) {
           return Ld{R2{ld32(A.vx, g), ld32(A.vy, g)}, Pol::MIXED ? ld32(d.f_cxy, g) : 0,
-                    ld32(reinterpret_cast<const int *>(A.cum), g)};
+                    CACHED ? 0 : ld32(reinterpret_cast<const int *>(A.cum), g)};
         },
         [&](int l, const Ld &v, int) {
           if constexpr (Pol::MIXED)  // tile frame, scaled units
             s_pos[l] = R2{kfma(v.pos.x, gs, xo), kfma((float)(((v.pk & 0xffff) >> 1) - gcy), fdy, v.pos.y) * gs};
           else
             s_pos[l] = v.pos;
-          dmax = max(dmax, v.cum);
+          if (!CACHED) dmax = max(dmax, v.cum);
         });
-    if (t < 4) s_pos[P.total + t] = R2{R(1e18), R(1e18)};
+    if (CACHED && far)  // (after the staging's loads, which do not wait for the flags)
+      for (int a = 0; a < P.nsc; ++a)
+        for (int q = t; q < P.len[a]; q += BLOCK)
+          dmax = max(dmax, ld32(reinterpret_cast<const int *>(A.cum), P.lo[a] + q));
+    if (CACHED && t < PADS) {  // the entries after each span
+      const int a = t / kRunPad<Pol>;
+      if (a < P.nsc) {
+        int b = PAD * a + t % kRunPad<Pol>;
+        for (int q = 0; q <= a; ++q) b += P.len[q];
+        s_pos[b] = R2{R(1e18), R(1e18)};
+      }
+    }
+    if (t < 4) s_pos[total + t] = R2{R(1e18), R(1e18)};
   }
   // walls: staged after the fluid candidates' padding
   const WallSpans W = wall_spans(d, P, cp);
-  const int wbase = P.total + 4;
+  const int wbase = total + 4;
   const bool wstaged = staged && W.n > 0 && P.total + W.n <= CAP + WCAP && W.nwr <= WROWS;
   if (wstaged) {
     const R fdx = cp.cdx_r, fdy = cp.cdy_r, gs = cp.gscale;
@@ -2480,17 +2532,22 @@ __global__ void __launch_bounds__(BLOCK, (MODE == kShiftCached ? 8 : 7))
     });
     if (t < 4) s_pos[wbase + W.n + t] = R2{R(1e18), R(1e18)};
   }
-  for (int o = 32; o > 0; o >>= 1) dmax = max(dmax, __shfl_xor(dmax, o, 64));
-  if ((t & 63) == 0) s_dmax[t >> 6] = __int_as_float(dmax);
-  __syncthreads();
-  float D = staged_bound<BLOCK>(s_dmax), Dsp = 0.f;
-  if constexpr (MODE == kShiftRecord) {
-    if (t == 0) d.tile_d0[tile] = D;
-  } else if constexpr (MODE == kShiftCached) {  // the staged paths count from the first pass
-    Dsp = D;
-    D = d.tile_d0[tile] + Dsp;
+  float d0 = 0.f;
+  if constexpr (CACHED) d0 = d.tile_d0[tile];
+  if (!CACHED || far) {
+    for (int o = 32; o > 0; o >>= 1) dmax = max(dmax, __shfl_xor(dmax, o, 64));
+    if ((t & 63) == 0) s_dmax[t >> 6] = __int_as_float(dmax);
   }
-  shift_tile<Pol, BLOCK, MODE, int, WROWS>(d, P, pass, own, s_pos, s_lb, s_wlb, D, Dsp, staged && use_runs, staged,
+  __syncthreads();
+  float D, Dsp = 0.f;
+  if constexpr (CACHED) {  // the staged paths count from the first pass
+    Dsp = far ? staged_bound<BLOCK>(s_dmax) : 0.5f * cp.skin_ok;
+    D = d0 + Dsp;
+  } else {
+    D = staged_bound<BLOCK>(s_dmax);
+    if (MODE == kShiftRecord && t == 0) d.tile_d0[tile] = D;
+  }
+  shift_tile<Pol, BLOCK, MODE, WROWS>(d, P, pass, own, s_pos, s_lb, s_wlb, D, Dsp, staged && use_runs, staged,
                                            wstaged, W);
 }
 

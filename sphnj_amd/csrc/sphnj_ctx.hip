@@ -400,6 +400,7 @@ struct Engine : EngineBase {
     d.nf = nf;
     d.ns = ns;
     d.nw = nw;
+    d.ncol = G / 2;
     CaseDev<R> *cases;
     int *fco, *sco, *wco;
     if ((rc = dalloc(&cases, ncase)) || (rc = dalloc(&fco, ncase + 1)) || (rc = dalloc(&sco, ncase + 1)) ||
@@ -464,7 +465,7 @@ struct Engine : EngineBase {
         (rc = dalloc(&cnt_toff, (size_t)nblk(4 * nc, kScanTile) + 1)) ||
         (rc = dalloc(&d.f_col, nf)) || (rc = dalloc(&d.f_near, nf)) || (rc = dalloc(&d.f_L, 4 * (size_t)nf)) ||
         (rc = dalloc(&d.f_sacc, 2 * (size_t)nf)) || (rc = dalloc(&d.f_wc, nf)) ||
-        (rc = dalloc(&d.tile_d0, (size_t)max_tiles(64))) ||
+        (rc = dalloc(&d.tile_d0, (size_t)max_tiles(64))) || (rc = dalloc(&d.f_far, (size_t)G)) ||
         (rc = dalloc(&d.f_srange, 4 * (size_t)nc)) || (rc = dalloc(&d.umax2, ncase)) || (rc = dalloc(&d.umax, ncase)) ||
         (rc = dalloc(&d.umax_slot, (size_t)ncase * kSpread * kSlotStride)) || (rc = dalloc(&d.status, 1)) ||
         (rc = dalloc(&d.u2_last, ncase)) || (rc = dalloc(&d.dtv, ncase)) || (rc = dalloc(&d.tsim, ncase)) ||
@@ -527,6 +528,7 @@ struct Engine : EngineBase {
     }
     HIPC(hipMemsetAsync(d.f_cnt, 0, (4 * (size_t)nc + 1) * sizeof(int), stream));  // zero between steps
     HIPC(hipMemsetAsync(d.f_srange, 0, 4 * (size_t)nc * sizeof(int2), stream));
+    HIPC(hipMemsetAsync(d.f_far, 0, (size_t)G * sizeof(int), stream));
 
     // ---- solid
     if ((rc = dalloc(&d.sx, ns)) || (rc = dalloc(&d.sy, ns)) || (rc = dalloc(&d.su, ns)) || (rc = dalloc(&d.sv, ns)) ||
@@ -1027,6 +1029,7 @@ struct Engine : EngineBase {
             if (rc) return rc;
             swap_shift_buffers();
           }
+          pair_runs = false;  // the recorded runs and the column flags serve these passes only
         }
         return SPHNJ_OK;
     }
