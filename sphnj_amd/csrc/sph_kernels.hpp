@@ -2721,17 +2721,23 @@ __device__ __forceinline__ void solid_deform_body(const Dev<Pol> &d, int sub, in
   using R = typename Pol::R;
   const int i = gid / kSolidLanes, l = gid % kSolidLanes;
   const bool active = i < d.ns;
-  int c = 0;
+  int c = 0, mat = 0, degen = 0;
   R h00 = 0, h01 = 0, h10 = 0, h11 = 0;
+  Mat2<R> L = {0, 0, 0, 0};
   if (active) {
     c = case_of(i, d.s_case_off, d.s_case_blk, d.ncase);
+    // (read here with the particle's other data, not after the sums: one wait on memory less)
+    const R *Lr = d.s_Lref + 4 * i;
+    L = {Lr[0], Lr[1], Lr[2], Lr[3]};
+    mat = d.s_mat[i];
+    degen = d.s_degen[i];
     if (sub < d.cases[c].S) {
       const double dix = d.sx[i] - d.sX[i], diy = d.sy[i] - d.sY[i];
       struct Nb {
         R gX, gY;
         double x, X, y, Y;
       };
-      for_refs<4>(
+      for_refs<2>(
           d.s_ref_j, d.s_ref_off[i] + l, d.s_ref_off[i + 1],
           [&](int e, int j) { return Nb{d.s_ref_g[2 * e], d.s_ref_g[2 * e + 1], d.sx[j], d.sX[j], d.sy[j], d.sY[j]}; },
           [&](int, int, const Nb &n) {
@@ -2750,10 +2756,8 @@ __device__ __forceinline__ void solid_deform_body(const Dev<Pol> &d, int sub, in
   if (!active || l != 0) return;
   const auto &cp = d.cases[c];
   if (sub >= cp.S) return;
-  const R *Lr = d.s_Lref + 4 * i;
-  const Mat2<R> L = {Lr[0], Lr[1], Lr[2], Lr[3]};
   Mat2<R> H;
-  if (d.s_degen[i]) {  // det(B) == 0: L = I, F = B + H~
+  if (degen) {  // det(B) == 0: L = I, F = B + H~
     const R *Bt = d.s_Bt + 4 * i;
     H = {Bt[0] + h00 - R(1), Bt[1] + h01, Bt[2] + h10, Bt[3] + h11 - R(1)};
   } else {
@@ -2765,7 +2769,6 @@ __device__ __forceinline__ void solid_deform_body(const Dev<Pol> &d, int sub, in
   const R e11 = H.d + R(0.5) * (H.b * H.b + H.d * H.d);
   const R e01 = R(0.5) * (H.b + H.c + H.a * H.b + H.c * H.d);
   Mat2<R> P = {0, 0, 0, 0};
-  const int mat = d.s_mat[i];
   R *Mp = d.s_M + 4 * i;
   if (mat == 0) {  // LINEAR_ELASTIC = St Venant-Kirchhoff (linearStressCalculation)
     const R trE = e00 + e11;
@@ -2825,47 +2828,85 @@ __device__ __forceinline__ void solid_deform_body(const Dev<Pol> &d, int sub, in
   o[3] = PL.d;
 }
 
+// Fluid -> solid Riemann force of a sub-step (solidFluidCouple, src/solid.cu:211-255:
+// rho_i = rho_j, u_i = u_s, p_i = p_s, c = c[phase_j]) into s_cp.  It reads the solids' positions
+// and velocities and the fluid, none of which the deformation writes, so the two share a launch:
+// apart, the force kernel summed the fluid and then the reference list one after the other, each a
+// chain of dependent loads.  A sub-step's two launches together, before -> with the fluid's force
+// beside the deformation -> with its candidates in neighbouring lanes: 395 solids P64 14.3 -> 12.9
+// -> 9.8 us, 8.3 k solids 17.9 -> 17.6 -> 15.6 (P64), 22.2 -> 20.0 -> 15.7 (M32).
 template <class Pol>
-__global__ void __launch_bounds__(256) k_solid_deform(Dev<Pol> d, int sub) {
-  solid_deform_body(d, sub, (int)(blockIdx.x * blockDim.x + threadIdx.x));
-}
-
-// solidForceCalculate (src/solid.cu:307-353: solidFluidCouple :211-255, solidSolidForce
-// :257-305) fused with solidUpdate (:446-471); positions and velocities ping-pong.
-template <class Pol>
-__device__ __forceinline__ void solid_force_body(const Dev<Pol> &d, int sub, int gid) {
+__device__ __forceinline__ void solid_fluid_body(const Dev<Pol> &d, int sub, int gid) {
   using R = typename Pol::R;
+  constexpr int kSpans = 6, kU = 6;
   const int i = gid / kSolidLanes, l = gid % kSolidLanes;
-  const bool active = i < d.ns;
-  int c = 0;
-  bool run = false;
-  R cpx = 0, cpy = 0, ax = 0, ay = 0;
-  if (active) {
-    c = case_of(i, d.s_case_off, d.s_case_blk, d.ncase);
+  bool run = i < d.ns;
+  R cpx = 0, cpy = 0;
+  if (run) {
+    const int c = case_of(i, d.s_case_off, d.s_case_blk, d.ncase);
     const auto &cp = d.cases[c];
     run = sub < cp.S;
     if (run) {
       const int pk = d.s_cxy[i], cx = cxy_x(pk), cy = cxy_y(pk);
-      const double xi = d.sx[i], yi = d.sy[i], ui = d.su[i], vi = d.sv[i];
-      const int mat = d.s_mat[i];
-      const R rr_inv = mat == 1 ? cp.rho_aux_inv : cp.rho_s_inv;
+      const double xi = d.sx[i], yi = d.sy[i];
+      const R rr_inv = d.s_mat[i] == 1 ? cp.rho_aux_inv : cp.rho_s_inv;
       const LoopConsts<R> K(cp);
-      // fluid -> solid Riemann force (rho_i = rho_j, u_i = u_s, p_i = p_s, c = c[phase_j])
       const R xiv = view_x<Pol>(xi, cx, cp), yiv = view_y<Pol>(yi, cy, cp);
-      const R uiv = (R)ui, viv = (R)vi, psi = d.s_p[i];
+      const R uiv = (R)d.su[i], viv = (R)d.sv[i], psi = d.s_p[i];
       const R c0 = cp.c[0], c1 = cp.c[1];
       const auto &F = d.fa;
-      // the 3x3 cells' 18 fluid runs (one per sub-column of a cell) go to the group's lanes,
-      // each lane summing its runs in slot order: the lanes read their runs' ranges together
-      // instead of the group walking the cells one after another
-      for (int r = l; r < kCellRuns; r += kSolidLanes) {
-        int2 rr;
+      // The 3x3 cells' fluid is one span of slots per sub-column: six spans, whose ends lanes
+      // 0..5 read from the row table.  The group walks them as one list, lane l taking entries
+      // l, l + kSolidLanes, ...: its lanes read neighbouring slots, where a lane per run of a cell
+      // had 64 lanes of a wave in 64 different lines.
+      const int sx = 2 * (cx - 1) + l, ny2 = 2 * cp.ny;
+      int lo = 0, len = 0;
+      if (l < kSpans && sx >= 0 && sx < 2 * cp.nx && d.nf > 0) {
+        const int *lb = d.f_lb + cp.lb_off + sx * (ny2 + 1);
+        lo = lb[max(2 * (cy - 1), 0)];
+        len = lb[min(2 * (cy + 2), ny2)] - lo;
+      }
+      // slot - entry of span 0, then its growth from span to span; the first entry after a span
+      int off[kSpans], end[kSpans], n_ = 0, o_ = 0;
+#pragma unroll
+      for (int a = 0; a < kSpans; ++a) {
+        const int o = __shfl(lo, a, kSolidLanes) - n_;
+        off[a] = o - o_;
+        o_ = o;
+        n_ += __shfl(len, a, kSolidLanes);
+        end[a] = n_;
+      }
+      const int n = end[kSpans - 1];
+      struct Nb {
+        FluidNb<R> f;
         R bx, by;
-        if (!cell_run(d, cp, cx, cy, r, xiv, yiv, rr, bx, by)) continue;
-        for_run<4>(rr.x, rr.y, [&](int s) { return FluidNb<R>::load(F, d.f_phase, s); }, [&](int, const FluidNb<R> &f) {
-          const R dx = f.x - bx, dy = f.y - by;
+      };
+      auto load = [&](int e) {
+        int o = off[0], a = -1;
+#pragma unroll
+        for (int k = 1; k < kSpans; ++k) {
+          const bool in = e >= end[k - 1];
+          o += in ? off[k] : 0;
+          a += in && !(k & 1) ? 1 : 0;
+        }
+        const int s = o + e;
+        Nb v;
+        v.f = FluidNb<R>::load(F, d.f_phase, s);
+        v.bx = xiv - cell_shift_x<Pol>(a, cp);
+        v.by = yiv - cell_shift_y<Pol>(Pol::MIXED ? (cxy_y(d.f_cxy[s]) >> 1) - cy : 0, cp);
+        return v;
+      };
+      for (int e0 = l; e0 < n; e0 += kU * kSolidLanes) {
+        Nb v[kU];
+#pragma unroll
+        for (int u = 0; u < kU; ++u) v[u] = load(min(e0 + u * kSolidLanes, n - 1));
+#pragma unroll
+        for (int u = 0; u < kU; ++u) {
+          if (e0 + u * kSolidLanes >= n) continue;
+          const FluidNb<R> &f = v[u].f;
+          const R dx = f.x - v[u].bx, dy = f.y - v[u].by;
           const R r2 = dx * dx + dy * dy;
-          if (!(r2 < K.rc2)) return;
+          if (!(r2 < K.rc2)) continue;
           const R w = K.w(r2);
           const R inv_r = r2 > R(0) ? krsqrt<R>(r2) : R(0);
           R ps = R(0.5) * (f.p + psi);
@@ -2874,8 +2915,54 @@ __device__ __forceinline__ void solid_force_body(const Dev<Pol> &d, int sub, int
           const R t = R(-2) * ps * rr_inv * w;
           cpx += t * dx;
           cpy += t * dy;
-        });
+        }
       }
+    }
+  }
+  cpx = group_sum(cpx);
+  cpy = group_sum(cpy);
+  if (!run || l != 0) return;
+  d.s_cp[2 * i] = cpx;
+  d.s_cp[2 * i + 1] = cpy;
+}
+
+// Blocks below half sum the fluid's force, the others the deformation.
+template <class Pol>
+__global__ void __launch_bounds__(256) k_solid_deform(Dev<Pol> d, int sub, int half) {
+  const int b = (int)blockIdx.x;
+  if (b < half)
+    solid_fluid_body(d, sub, b * 256 + (int)threadIdx.x);
+  else
+    solid_deform_body(d, sub, (b - half) * 256 + (int)threadIdx.x);
+}
+
+// solidSolidForce (src/solid.cu:257-305) and, with the fluid's force, solidUpdate (:446-471);
+// positions and velocities ping-pong.
+template <class Pol>
+__device__ __forceinline__ void solid_force_body(const Dev<Pol> &d, int sub, int gid) {
+  using R = typename Pol::R;
+  const int i = gid / kSolidLanes, l = gid % kSolidLanes;
+  const bool active = i < d.ns;
+  int c = 0, pk = 0, bc = 0;
+  bool run = false;
+  R cpx = 0, cpy = 0, ax = 0, ay = 0;
+  double xi = 0, yi = 0, ui = 0, vi = 0, dtc = 0;
+  if (active) {
+    c = case_of(i, d.s_case_off, d.s_case_blk, d.ncase);
+    const auto &cp = d.cases[c];
+    run = sub < cp.S;
+    if (run) {
+      // (all of the particle's data at once, what the update needs included)
+      pk = d.s_cxy[i];
+      bc = d.s_bc[i];
+      cpx = d.s_cp[2 * i];
+      cpy = d.s_cp[2 * i + 1];
+      dtc = d.dtv[c];
+      xi = d.sx[i];
+      yi = d.sy[i];
+      ui = d.su[i];
+      vi = d.sv[i];
+      const R rr_inv = d.s_mat[i] == 1 ? cp.rho_aux_inv : cp.rho_s_inv;
       // solid -> solid over the reference-configuration list
       const R *Fi = d.s_F + 4 * i, *Li = d.s_L + 4 * i, *PLi = d.s_PL + 4 * i;
       const Mat2<R> FL = mmul(Mat2<R>{Fi[0], Fi[1], Fi[2], Fi[3]}, Mat2<R>{Li[0], Li[1], Li[2], Li[3]});
@@ -2885,7 +2972,7 @@ __device__ __forceinline__ void solid_force_body(const Dev<Pol> &d, int sub, int
         R gX, gY, p0, p1, p2, p3;
         double x, y, u, v;
       };
-      for_refs<4>(
+      for_refs<2>(
           d.s_ref_j, d.s_ref_off[i] + l, d.s_ref_off[i + 1],
           [&](int e, int j) {
             const R *PLj = d.s_PL + 4 * j;
@@ -2904,8 +2991,6 @@ __device__ __forceinline__ void solid_force_body(const Dev<Pol> &d, int sub, int
           });
     }
   }
-  cpx = group_sum(cpx);
-  cpy = group_sum(cpy);
   ax = group_sum(ax);
   ay = group_sum(ay);
   if (!active || l != 0) return;
@@ -2921,14 +3006,11 @@ __device__ __forceinline__ void solid_force_body(const Dev<Pol> &d, int sub, int
     }
     return;
   }
-  const int pk = d.s_cxy[i], cx = cxy_x(pk), cy = cxy_y(pk);
-  const double xi = d.sx[i], yi = d.sy[i], ui = d.su[i], vi = d.sv[i];
-  const double dt_s = d.dtv[c] / (double)cp.S;  // solid sub-step (src/solid.cu:456)
-  d.s_cp[2 * i] = cpx;
-  d.s_cp[2 * i + 1] = cpy;
+  const int cx = cxy_x(pk), cy = cxy_y(pk);
+  const double dt_s = dtc / (double)cp.S;  // solid sub-step (src/solid.cu:456)
   double tax = (double)ax + (double)cpx, tay = (double)ay + (double)cpy;
   double x = xi, y = yi, u = ui, v = vi;
-  if (d.s_bc[i] == 1) {  // FIXED_PARTICLE
+  if (bc == 1) {  // FIXED_PARTICLE
     u = cp.fixed_u;
     v = cp.fixed_v;
     x += u * dt_s;
@@ -3025,6 +3107,8 @@ __global__ void __launch_bounds__(kSubstepBlock) k_solid_substeps(Dev<Pol> d0, D
   unsigned e = 0;
   for (int k = 0; k < S; ++k) {
     const Dev<Pol> &d = (k & 1) ? d1 : d0;
+    for (int gid = blockIdx.x * blockDim.x + threadIdx.x; gid - (int)threadIdx.x < n; gid += stride)
+      solid_fluid_body(d, k, gid);
     for (int gid = blockIdx.x * blockDim.x + threadIdx.x; gid - (int)threadIdx.x < n; gid += stride)
       solid_deform_body(d, k, gid);
     grid_sync(g, ++e, spin_limit, d0.status);

@@ -1009,8 +1009,9 @@ struct Engine : EngineBase {
           }
           for (int k = 0; k < S; ++k) {
             if (!one) {
-              k_solid_deform<Pol><<<nblk(ns * kSolidLanes, 256), 256, 0, stream>>>(d, k);
-              k_solid_force_update<Pol><<<nblk(ns * kSolidLanes, 256), 256, 0, stream>>>(d, k);
+              const int nb = nblk(ns * kSolidLanes, 256);
+              k_solid_deform<Pol><<<2 * nb, 256, 0, stream>>>(d, k, nb);
+              k_solid_force_update<Pol><<<nb, 256, 0, stream>>>(d, k);
               LAUNCH_CHECK();
             }
             std::swap(d.sx, d.sx2);
