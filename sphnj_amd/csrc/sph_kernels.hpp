@@ -559,6 +559,7 @@ template <class Pol, int kWallLanes>
 __device__ __forceinline__ void wall_update_block(const Dev<Pol> &d, int bid) {
   using R = typename Pol::R;
   constexpr int NP = kWallPartials / kWallLanes;  // partial sums per lane
+  constexpr int kRuns = (kCellRuns + kWallPartials - 1) / kWallPartials, kU = 4;
   static_assert(NP * kWallLanes == kWallPartials, "group size divides the partial count");
   const int gid = bid * 256 + (int)threadIdx.x;
   const int i = gid / kWallLanes, l = gid % kWallLanes;
@@ -577,27 +578,41 @@ __device__ __forceinline__ void wall_update_block(const Dev<Pol> &d, int bid) {
     // the 3x3 cells' 18 fluid runs: partial sum k = l + j * LANES takes runs k, k + 8, ...
 #pragma unroll
     for (int j = 0; j < NP; ++j) {
-      for (int r = l + j * kWallLanes; r < kCellRuns; r += kWallPartials) {
-        int2 rr;
-        R bx, by;
-        if (!cell_run(d, cp, cx, cy, r, xi, yi, rr, bx, by)) continue;
-        for (int s = rr.x; s < rr.y; ++s) {
-          const R dx = F.vx[s] - bx, dy = F.vy[s] - by;
-          const R r2 = dx * dx + dy * dy;
-          if (!(r2 < cp.rc2)) continue;
-          const R w = (kgauss2<R>(r2, cp.hinv2, cp.nhl2) - cp.eR) * cp.k2c;
-          S[j] += w;
-          U[j] += F.vu[s] * w;
-          V[j] += F.vv[s] * w;
-          P[j] += (F.p[s] - F.vrho[s] * (cp.gx * dx + cp.gy * dy)) * w;
-          // first strict minimum of the serial scan: ties go to the earlier run
-          if (near_run == kCellRuns || r2 < nearest || (r2 == nearest && r < near_run)) {
-            near_run = r;
-            nearest = r2;
-            phase = d.f_phase[s];
-          }
-        }
+      // their ranges together, then as one list kU candidates together with all of their fields: a
+      // candidate at a time, its position first, was some twenty dependent waits a wall
+      const int r0 = l + j * kWallLanes;
+      int lo[kRuns], end[kRuns], n = 0;
+      R bx[kRuns], by[kRuns];
+#pragma unroll
+      for (int q = 0; q < kRuns; ++q) {
+        const int r = r0 + q * kWallPartials;
+        int2 rr = {0, 0};
+        bx[q] = by[q] = 0;
+        if (r < kCellRuns && !cell_run(d, cp, cx, cy, r, xi, yi, rr, bx[q], by[q])) rr = {0, 0};
+        lo[q] = rr.x - n;
+        end[q] = n += max(rr.y - rr.x, 0);
       }
+      auto of = [&](int e, auto a0, auto a1, auto a2) { return e < end[0] ? a0 : (e < end[1] ? a1 : a2); };
+      static_assert(kRuns == 3, "of() picks one of three");
+      for_run<kU>(
+          0, n, [&](int e) { return FluidNb<R>::load(F, d.f_phase, of(e, lo[0], lo[1], lo[2]) + e); },
+          [&](int e, const FluidNb<R> &f) {
+            const R dx = f.x - of(e, bx[0], bx[1], bx[2]), dy = f.y - of(e, by[0], by[1], by[2]);
+            const R r2 = dx * dx + dy * dy;
+            if (!(r2 < cp.rc2)) return;
+            const R w = (kgauss2<R>(r2, cp.hinv2, cp.nhl2) - cp.eR) * cp.k2c;
+            S[j] += w;
+            U[j] += f.u * w;
+            V[j] += f.v * w;
+            P[j] += (f.p - f.rho * (cp.gx * dx + cp.gy * dy)) * w;
+            // first strict minimum of the serial scan: ties go to the earlier run
+            const int r = r0 + of(e, 0, 1, 2) * kWallPartials;
+            if (near_run == kCellRuns || r2 < nearest || (r2 == nearest && r < near_run)) {
+              near_run = r;
+              nearest = r2;
+              phase = f.phase;
+            }
+          });
     }
   }
   // the butterfly's levels 4, 2, ... that pair partials of one lane, then those across lanes
@@ -942,7 +957,7 @@ __device__ __forceinline__ void subcol_rows_block(const Dev<Pol> &d, int G, cons
     if (__ballot(over ? 1 : 0) != 0ull && lane == 0) atomicOr(d.status, kStCellOver64);
   }
   if (w == 2 % NW && d.ns > 0) {  // ... and builds its f_swp
-    constexpr int kU = 8;
+    constexpr int kU = 4;
     const int qc = cp.cell_off + (sx >> 1) * cp.ny;
     int *swp = d.f_swp + cp.swp_off + (sx >> 1) * (cp.ny + 1);
     const int pc = (cp.ny + 63) >> 6, c0 = min(lane * pc, cp.ny), c1 = min(c0 + pc, cp.ny);
