@@ -170,6 +170,10 @@ struct Dev {
   int *w_lb;
   // status word (SPHNJ_ST_* bits)
   unsigned *status;
+  // P64: per slot, the walls within reach when the runs were recorded (WallList; quads nf apart).
+  // Last: the fields before it stay where their wide scalar loads are aligned (eight bytes ahead of
+  // them cost a M32 shift pass 4 %)
+  uint4 *f_wl;
 };
 
 // ---- helpers ----------------------------------------------------------------------------

@@ -579,7 +579,8 @@ __device__ __forceinline__ void wall_update_block(const Dev<Pol> &d, int bid) {
 #pragma unroll
     for (int j = 0; j < NP; ++j) {
       // their ranges together, then as one list kU candidates together with all of their fields: a
-      // candidate at a time, its position first, was some twenty dependent waits a wall
+      // candidate at a time, its position first, was some twenty dependent waits a wall (a step of
+      // 5 k particles 183.5 -> 181 us; eight at a time cost registers: a 320 k tank 970 -> 974)
       const int r0 = l + j * kWallLanes;
       int lo[kRuns], end[kRuns], n = 0;
       R bx[kRuns], by[kRuns];
@@ -1425,6 +1426,42 @@ __device__ __forceinline__ float staged_bound(const float *s_dmax) {
   return D * (1.0f + 1e-6f);
 }
 
+// A lane's recorded wall candidates: the walls of its 3x3 cells within rc (1 + s) at the recording,
+// by their place in the tile's wall list and in the order the neighbour loops take them, one byte
+// each.  Byte 0 holds 1 + the number of bytes in use, itself included (0: no list -- the tile's walls
+// are not staged, more than 255, or the lane has more than kWallListBytes - 1); bytes past the last are
+// the tile's padding entry.  Word w of a lane is component w % 4 of f_wl[(w / 4) nf + slot].
+//   A lane beside a wall has 36 to 77 walls in its 3x3 cells and 15 to 25 of them within reach;
+// walked whole they took a third of a P64 pass's slowest wave on a 5 k particle dam break, whose
+// blocks have a CU each.  From the lists its step takes 240 instead of 259 us, that of 800 particles
+// 245 instead of 262, of a 93 k two-phase flow 375 instead of 381; 3.0 M particles 3.41 ms as before.
+// M32 walks its walls whole: a term costs it no more than a list entry's decoding, and the recording
+// cost the pair kernel more than the passes gained (187 k two-phase flow 276 -> 284 us per step).
+constexpr int kWallListQuads = 3, kWallListBytes = 16 * kWallListQuads;
+template <class Pol>
+constexpr bool kWallLists = !Pol::MIXED;
+struct WallList {
+  int n;  // bytes in use; 0: no list
+  __device__ __forceinline__ explicit WallList(int walls) : n(walls <= 255 ? 1 : 0) {}
+  __device__ __forceinline__ static void byte(uint4 *f_wl, int nf, int i, int k, unsigned v) {
+    reinterpret_cast<uint8_t *>(f_wl + (size_t)(k >> 4) * nf + i)[k & 15] = (uint8_t)v;
+  }
+  // the walls b + k, bit k of m set
+  __device__ __forceinline__ void put(uint4 *f_wl, int nf, int i, int b, unsigned m) {
+    if (n + __builtin_popcount(m) > kWallListBytes) n = 0;
+    if (n == 0) return;
+#pragma unroll 1
+    for (; m; m &= m - 1u) byte(f_wl, nf, i, n++, (unsigned)(b + __builtin_ctz(m)));
+  }
+  // pad: the tile's padding entry
+  __device__ __forceinline__ void close(uint4 *f_wl, int nf, int i, int pad) {
+    if (n > 0)
+      for (int k = n; k & 3; ++k) byte(f_wl, nf, i, k, (unsigned)pad);  // to a whole word
+    byte(f_wl, nf, i, 0, n > 0 ? (unsigned)n + 1u : 0u);
+  }
+  __device__ __forceinline__ static void none(uint4 *f_wl, int i) { byte(f_wl, 0, i, 0, 0u); }
+};
+
 // Calls f(s) for s in [lo, hi), U at a time so the loads of U candidates are in flight together.
 template <int U, class F>
 __device__ __forceinline__ void for_range(int lo, int hi, F &&f) {
@@ -2001,17 +2038,23 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
         // column beside a side wall holds about 47, of which some 20 lie inside the cut-off;
         // evaluated whole they made the walls' waves the slowest of a launch)
         const int lr0 = max(cy - 1, 0) - W.wcr0, lr1 = min(cy + 1, cp.ny - 1) - W.wcr0;
+        // (a recording also lists the walls within rc (1 + s), in this order, for the shift passes)
+        WallList wl(W.n);
 #pragma unroll 1
         for (int a = 0; a < 3; ++a) {
           const int s0 = s_wlb[a][lr0], s1 = s_wlb[a][lr1 + 1];
 #pragma unroll 1
           for (int b = s0; b < s1; b += 32) {
             unsigned ms;
-            eval2(mark(std::false_type{}, b, min(b + 32, s1), ms), b, 0u, 0, s1 - s0 > 32);
+            const unsigned m = mark(std::bool_constant<kWallLists<Pol>>{}, b, min(b + 32, s1), ms);
+            if (kWallLists<Pol> && record) wl.put(d.f_wl, d.nf, i, b - wbase, ms);
+            eval2(m, b, 0u, 0, s1 - s0 > 32);
           }
         }
+        if (kWallLists<Pol> && record) wl.close(d.f_wl, d.nf, i, W.n);
       }
     }
+    if (kWallLists<Pol> && record && (P.sw & 1) && !wstaged) WallList::none(d.f_wl, i);
     for_windows<true>(P, cp, lsx, sy, cy, lp, Rp, [&](int sc, int ra, int rb) {
       if (staged) return;
       const R bx = xi - cell_shift_x<Pol>((sc >> 1) - cx, cp);
@@ -2156,6 +2199,7 @@ struct ShiftOwn {
   R2 sacc{R(0), R(0)};
   float cum0 = 0.f, cum_hash = 0.f;
   uint3 wc{0u, 0u, 0u};
+  uint4 wl{0u, 0u, 0u, 0u};
 };
 template <class Pol, int MODE>
 __device__ __forceinline__ ShiftOwn<Pol> shift_own(const Dev<Pol> &d, const TilePlan &P, int pass, int K) {
@@ -2180,6 +2224,7 @@ __device__ __forceinline__ ShiftOwn<Pol> shift_own(const Dev<Pol> &d, const Tile
       if constexpr (MODE == kShiftCached) {
         o.wc = *reinterpret_cast<const uint3 *>(d.f_wc + i);
         if (lastp) o.cum_hash = __uint_as_float(d.f_wc[i].w);
+        if (kWallLists<Pol> && (P.sw & 1)) o.wl = d.f_wl[i];
       }
     }
   }
@@ -2196,7 +2241,7 @@ __device__ __forceinline__ void shift_tile(const Dev<Pol> &d, const TilePlan &P,
                                            const typename V2<typename Pol::R>::T *s_pos,
                                            const int (*s_lb)[TileRows<BLOCK>::value + 1], const int (*s_wlb)[WROWS + 1],
                                            float D, float Dsp, bool runs, bool staged, bool wstaged,
-                                           const WallSpans &W) {
+                                           const WallSpans &W, int wbase) {
 #pragma clang fp contract(off)
   using R = typename Pol::R;
   using R2 = typename V2<R>::T;
@@ -2344,9 +2389,26 @@ __device__ __forceinline__ void shift_tile(const Dev<Pol> &d, const TilePlan &P,
       }
     });
   }
-  if constexpr (MODE == kShiftRecord) d.f_wc[i] = rr.entry(cum0);
+  if constexpr (MODE == kShiftRecord) {
+    d.f_wc[i] = rr.entry(cum0);
+    if (kWallLists<Pol> && (P.sw & 1)) WallList::none(d.f_wl, i);
+  }
   // walls of the 3x3 cells (cell column by cell column, rows in order), then solids
-  if (wstaged) {
+  if (kWallLists<Pol> && wstaged && cached && (own.wl.x & 0xffu)) {  // those the recording listed, four to a word
+    const int words = ((int)(own.wl.x & 0xffu) + 2) >> 2;
+    uint4 q = own.wl, nx{0u, 0u, 0u, 0u};
+    q.x = (q.x & ~0xffu) | (unsigned)W.n;
+#pragma unroll 1
+    for (int w = 0; w < words; ++w) {
+      if ((w & 3) == 0 && w + 4 < words) nx = d.f_wl[(size_t)((w >> 2) + 1) * d.nf + i];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) (void)staged_term(wbase + (int)((q.x >> (8 * k)) & 0xffu));
+      q.x = q.y;
+      q.y = q.z;
+      q.z = q.w;
+      if ((w & 3) == 3) q = nx;
+    }
+  } else if (wstaged) {
     const int lr0 = max(cy - 1, 0) - W.wcr0, lr1 = min(cy + 1, cp.ny - 1) - W.wcr0;
 #pragma unroll
     for (int a = 0; a < 3; ++a) for_range_4_2_1(s_wlb[a][lr0], s_wlb[a][lr1 + 1], staged_add);
@@ -2563,7 +2625,7 @@ __global__ void __launch_bounds__(BLOCK, 7)
     if (MODE == kShiftRecord && t == 0) d.tile_d0[tile] = D;
   }
   shift_tile<Pol, BLOCK, MODE, WROWS>(d, P, pass, own, s_pos, s_lb, s_wlb, D, Dsp, staged && use_runs, staged,
-                                           wstaged, W);
+                                           wstaged, W, wbase);
 }
 
 // ======================================================================================
