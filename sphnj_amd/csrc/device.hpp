@@ -87,8 +87,11 @@ struct FluidBuf {
   float *cum;  // path length since the hash (sum of step lengths): bounds |x - x at hash|
 };
 
+// The order and the alignment count: the compiler reads the pointers in wide scalar loads where
+// they lie on multiples of them, and eight bytes more or less ahead of the others cost the M32 shift
+// and pair kernels 1 to 4 %.
 template <class Pol>
-struct Dev {
+struct alignas(16) Dev {
   using R = typename Pol::R;
   const CaseDev<R> *cases;
   int ncase;
@@ -99,15 +102,15 @@ struct Dev {
   // fluid
   FluidBuf<Pol> fa, fb;  // cur (a) / alt (b)
   int8_t *f_phase, *f_phase2, *f_cls, *f_cls2;  // cur / alt (swap in the permute only)
-  int *f_orig;           // slot -> global original index (sorted values)
+  int *f_orig;           // slot -> global original index (sorted values); alt: f_orig2, as f_phase
   int *f_cxy;            // slot -> (sx << 16) | sy, sub-cell coordinates (cx = sx >> 1)
   // counting sort on the sub-cell keys: per key (4 total_cells + 1) the slots hashed there this
   // step (zero between steps); per slot of the order being replaced its key and its rank among
-  // its key's slots in atomic order; per slot in atomic order the old slot, original index and
-  // key (atomic order only permutes the slots inside a key, so f_pkey holds the sorted keys)
+  // its key's slots in atomic order; the original indices of the slots in atomic order
   int *f_cnt;
   int *f_hkey, *f_hrank;
-  int *f_perm, *f_porig, *f_pkey;
+  int *f_orig2, *f_porig;
+  unsigned *status;  // status word (SPHNJ_ST_* bits)
   R *f_col;
   int8_t *f_near;
   R *f_L;  // 4 per slot
@@ -168,11 +171,7 @@ struct Dev {
   // per cell column (case offset swp_off), ny + 1 entries: first wall slot of cell row k or
   // later, the column's end last (walls are sorted by cell once)
   int *w_lb;
-  // status word (SPHNJ_ST_* bits)
-  unsigned *status;
-  // P64: per slot, the walls within reach when the runs were recorded (WallList; quads nf apart).
-  // Last: the fields before it stay where their wide scalar loads are aligned (eight bytes ahead of
-  // them cost a M32 shift pass 4 %)
+  // P64: per slot, the walls within reach when the runs were recorded (WallList; quads nf apart)
   uint4 *f_wl;
 };
 

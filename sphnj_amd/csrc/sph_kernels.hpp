@@ -289,42 +289,56 @@ __global__ void __launch_bounds__(1024) k_exscan_small(const int *in, int n, int
   if (t == 1023) out[n] = part[1023];
 }
 
-// Counting sort, step 3: each key's [start, end) slot range (empty: [0, 0)), in rounds of
-// kSortThreads consecutive keys; the counts are cleared for the next step.  The tile's first
-// slot comes from toff (the scanned tile sums), or, with up to kApplyPrefixMax tiles and
+// Counting sort, step 3: each key's [start, end) slot range (empty: [0, 0)); the counts are
+// cleared for the next step.  A wave takes kScanItems rounds of 64 consecutive keys, the loads of
+// all rounds first, and scans them by itself; the waves meet once, for their totals (a block scan
+// a round was two barriers each: 5.7 -> 4.6 us a launch for 5 k particles, 8.2 -> 5.7 for 3.0 M).  The tile's
+// first slot comes from toff (the scanned tile sums), or, with up to kApplyPrefixMax tiles and
 // toff == nullptr, from the block's own sum of the tile sums before it (no scan launch).
 constexpr int kApplyPrefixMax = 4096;
 __global__ void __launch_bounds__(kSortThreads) k_count_apply(int *cnt, int nk, const int *tsum, const int *toff,
                                                                int2 *range) {
-  __shared__ int tmp[4];
-  int run;
-  if (toff != nullptr) {
-    run = toff[blockIdx.x];
-  } else {
-    int before = 0;
-    for (int k = (int)threadIdx.x; k < (int)blockIdx.x; k += kSortThreads) before += tsum[k];
-    before = wave_sum(before);
-    if ((threadIdx.x & 63) == 0) tmp[threadIdx.x >> 6] = before;
-    __syncthreads();
-    run = tmp[0] + tmp[1] + tmp[2] + tmp[3];
-    __syncthreads();  // tmp is reused by the scans below
-  }
+  constexpr int NW = kSortThreads / 64;
+  __shared__ int s_before[NW], s_tot[NW];
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int k0 = blockIdx.x * kScanTile + w * (64 * kScanItems) + lane;  // round q: k0 + 64 q
+  int c[kScanItems];
+#pragma unroll
+  for (int q = 0; q < kScanItems; ++q) c[q] = k0 + 64 * q < nk ? cnt[k0 + 64 * q] : 0;
+  int before = 0;
+  if (toff == nullptr)
+    for (int k = t; k < (int)blockIdx.x; k += kSortThreads) before += tsum[k];
+  else if (t == 0)
+    before = toff[blockIdx.x];
+  before = wave_sum(before);
+  int st[kScanItems], tot = 0;  // first slot of each key, from the wave's first
+#pragma unroll
   for (int q = 0; q < kScanItems; ++q) {
-    const int k = blockIdx.x * kScanTile + q * kSortThreads + (int)threadIdx.x;
-    const int c = k < nk ? cnt[k] : 0;
-    int tot;
-    const int st = run + block_exscan256(c, tmp, &tot);
+    const int in = wave_incl_sum(c[q], lane);
+    st[q] = tot + in - c[q];
+    tot += __shfl(in, 63, 64);
+  }
+  if (lane == 0) {
+    s_before[w] = before;
+    s_tot[w] = tot;
+  }
+  __syncthreads();
+  int run = 0;
+#pragma unroll
+  for (int v = 0; v < NW; ++v) run += s_before[v] + (v < w ? s_tot[v] : 0);
+#pragma unroll
+  for (int q = 0; q < kScanItems; ++q) {
+    const int k = k0 + 64 * q, a = run + st[q];
     if (k < nk) {
-      range[k] = c > 0 ? make_int2(st, st + c) : make_int2(0, 0);
+      range[k] = c[q] > 0 ? make_int2(a, a + c[q]) : make_int2(0, 0);
       cnt[k] = 0;
     }
-    run += tot;
   }
 }
 
-// Counting sort, step 4: every slot to its place in atomic order, with its original index
-// and key (so f_pkey holds the sorted keys).  kCellRounds rounds of 256 slots per block,
-// the loads of all rounds first.
+// Counting sort, step 4: every slot's original index to the slot's place in atomic order, so
+// that a key's [start, end) holds the original indices of its slots.  kCellRounds rounds of 256
+// slots per block, the loads of all rounds first.
 template <class Pol>
 __global__ void __launch_bounds__(256) k_count_scatter(Dev<Pol> d) {
   constexpr int U = kCellRounds;
@@ -341,14 +355,8 @@ __global__ void __launch_bounds__(256) k_count_scatter(Dev<Pol> d) {
 #pragma unroll
   for (int u = 0; u < U; ++u) p[u] = d.f_srange[k[u]].x + r[u];
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const int s = s0 + 256 * u;
-    if (s < d.nf) {
-      d.f_perm[p[u]] = s;
-      d.f_porig[p[u]] = o[u];
-      d.f_pkey[p[u]] = k[u];
-    }
-  }
+  for (int u = 0; u < U; ++u)
+    if (s0 + 256 * u < d.nf) d.f_porig[p[u]] = o[u];
 }
 
 // fillSolidCellID (src/pair.cu:29-36); solids stay in original order, the key array is the
@@ -395,8 +403,10 @@ __global__ void __launch_bounds__(256) k_hash_wall(Dev<Pol> d, const double *x, 
 
 // The counting sort's last step fused with the gather of the fluid state into sorted order
 // (the zip permute of Fluid_List::sort, src/sort.cu:10-20 / include/particle.cuh:93-96): a
-// thread per scattered slot finds the slot's final place in its key and writes the particle
-// there; also rebuilds the views and resets the per-case maximum speed slots and the path
+// thread per slot of the old order finds the slot's final place in its key and writes the particle
+// there (reading in old order takes the key and the original index as they lie, where a thread per
+// scattered slot needed the old slot and the key scattered too: with the scatter 97 -> 92 us for
+// 3.0 M particles, 143 -> 126 for 4.5 M); also rebuilds the views and resets the per-case maximum speed slots and the path
 // lengths of this step.
 template <class Pol>
 __global__ void __launch_bounds__(256) k_permute_fluid(Dev<Pol> d) {
@@ -411,7 +421,7 @@ __global__ void __launch_bounds__(256) k_permute_fluid(Dev<Pol> d) {
   // counting sort, step 5: inside each key, slots in original-index order -- a slot's place is
   // its key's start plus the number of the key's slots with a smaller original index -- so the
   // order is (sub-column, sub-row, original index) whatever order the atomics took
-  const int k = d.f_pkey[i], o = d.f_porig[i], s = d.f_perm[i];
+  const int s = i, k = d.f_hkey[s], o = d.f_orig[s];
   // the particle's state is loaded before the rank loop, which does not need it
   const double x = d.fa.x[s], y = d.fa.y[s], u = d.fa.u[s], v = d.fa.v[s], rho = d.fa.rho[s];
   const auto p = d.fa.p[s];
@@ -429,7 +439,7 @@ __global__ void __launch_bounds__(256) k_permute_fluid(Dev<Pol> d) {
   d.fb.cum[t] = 0.f;
   d.f_phase2[t] = phase;
   d.f_cls2[t] = cls;
-  d.f_orig[t] = o;
+  d.f_orig2[t] = o;
   const int c = case_of(t, d.f_case_off, d.f_case_blk, d.ncase);
   const auto &cp = d.cases[c];
   unsigned fl = 0;

@@ -459,8 +459,8 @@ struct Engine : EngineBase {
     }
     if ((rc = dalloc(&d.f_phase, nf)) || (rc = dalloc(&d.f_phase2, nf)) || (rc = dalloc(&d.f_cls, nf)) ||
         (rc = dalloc(&d.f_cls2, nf)) || (rc = dalloc(&d.f_orig, nf)) || (rc = dalloc(&d.f_cxy, nf)) ||
-        (rc = dalloc(&d.f_hkey, nf)) || (rc = dalloc(&d.f_hrank, nf)) || (rc = dalloc(&d.f_perm, nf)) ||
-        (rc = dalloc(&d.f_cnt, 4 * (size_t)nc + 1)) || (rc = dalloc(&d.f_porig, nf)) || (rc = dalloc(&d.f_pkey, nf)) ||
+        (rc = dalloc(&d.f_hkey, nf)) || (rc = dalloc(&d.f_hrank, nf)) || (rc = dalloc(&d.f_orig2, nf)) ||
+        (rc = dalloc(&d.f_cnt, 4 * (size_t)nc + 1)) || (rc = dalloc(&d.f_porig, nf)) ||
         (rc = dalloc(&cnt_tsum, (size_t)nblk(4 * nc, kScanTile) + 1)) ||
         (rc = dalloc(&cnt_toff, (size_t)nblk(4 * nc, kScanTile) + 1)) ||
         (rc = dalloc(&d.f_col, nf)) || (rc = dalloc(&d.f_near, nf)) || (rc = dalloc(&d.f_L, 4 * (size_t)nf)) ||
@@ -765,6 +765,7 @@ struct Engine : EngineBase {
       LAUNCH_CHECK();
       swap_fluid_all();
       std::swap(d.f_phase, d.f_phase2);
+      std::swap(d.f_orig, d.f_orig2);
       std::swap(d.f_cls, d.f_cls2);
     }
     if (ns > 0) {
@@ -1402,9 +1403,11 @@ struct Engine : EngineBase {
       n = f_off[c + 1] - lo;
       k.resize(n);
       o.resize(n);
-      if (n && (rc = d2h(k.data(), d.f_pkey + lo, n))) return rc;  // the scatter's keys are the sorted keys
+      if (n && (rc = d2h(k.data(), d.f_cxy + lo, n))) return rc;
       if ((rc = d2h(o.data(), d.f_orig + lo, n)) || (rc = d2h(rg.data(), d.f_srange + 4 * (size_t)cp.cell_off, nb)))
         return rc;
+      HIPC(hipStreamSynchronize(stream));
+      for (int t = 0; t < n; ++t) k[t] = 4 * cp.cell_off + (int)((uint32_t)k[t] >> 16) * 2 * cp.ny + (k[t] & 0xffff);
     } else if (species == SPHNJ_SOLID) {
       lo = s_off[c];
       n = s_off[c + 1] - lo;
