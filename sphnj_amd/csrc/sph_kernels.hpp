@@ -140,6 +140,46 @@ __device__ __forceinline__ void for_run(int lo, int hi, Ld &&load, F &&use) {
   }
 }
 
+// The solids of the 3x3 cells around (cx, cy), cell column by cell column, rows in order, as one
+// list (a column's three cells are one span of the sorted solids): use(dx, dy, v) with the offset
+// from (xi, yi) and v = load(j).  The nine ranges are read together, then the solids U at a time: a
+// cell and a solid at a time, range, index and position were nine chains of dependent loads for
+// every lane of a tile near a solid (pair kernel: 24 k gate P64 65 -> 56 us, 4.5 M wedge 639 -> 621).
+// The shift passes, which read positions only, walk the cells one by one: this way they took longer
+// (a 320 k tank with 10 passes 972 -> 987 us per step).
+template <class Pol, int U, class CP, class R, class Ld, class F>
+__device__ __forceinline__ void for_cell_solids(const Dev<Pol> &d, const CP &cp, int cx, int cy, R xi, R yi, Ld &&load,
+                                                F &&use) {
+  int2 r[9];
+#pragma unroll
+  for (int q = 0; q < 9; ++q) {
+    const int jx = cx - 1 + q / 3, jy = cy - 1 + q % 3;
+    const bool in = jx >= 0 && jx < cp.nx && jy >= 0 && jy < cp.ny;
+    r[q] = d.s_range[cp.cell_off + min(max(jx, 0), cp.nx - 1) * cp.ny + min(max(jy, 0), cp.ny - 1)];
+    if (!in) r[q] = make_int2(0, 0);
+  }
+  int lo[3], end[3], n = 0;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) {
+    const int2 s = run_join(run_join(r[3 * a], r[3 * a + 1]), r[3 * a + 2]);
+    lo[a] = s.x - n;
+    end[a] = n += max(s.y - s.x, 0);
+  }
+  struct Nb {
+    R x, y, bx, by;
+    decltype(load(0)) v;
+  };
+  for_run<U>(
+      0, n,
+      [&](int e) {
+        const int a = e < end[0] ? 0 : (e < end[1] ? 1 : 2);
+        const int j = d.s_sorted[(a == 0 ? lo[0] : (a == 1 ? lo[1] : lo[2])) + e];
+        return Nb{d.s_vx[j], d.s_vy[j], xi - cell_shift_x<Pol>(a - 1, cp),
+                  yi - cell_shift_y<Pol>(Pol::MIXED ? cxy_y(d.s_cxy[j]) - cy : 0, cp), load(j)};
+      },
+      [&](int, const Nb &q) { use(q.x - q.bx, q.y - q.by, q.v); });
+}
+
 // Case owning global cell i (cases hold consecutive cell ranges).
 template <class Pol>
 __device__ __forceinline__ int case_of_cell(int i, const Dev<Pol> &d) {
@@ -406,8 +446,8 @@ __global__ void __launch_bounds__(256) k_hash_wall(Dev<Pol> d, const double *x, 
 // thread per slot of the old order finds the slot's final place in its key and writes the particle
 // there (reading in old order takes the key and the original index as they lie, where a thread per
 // scattered slot needed the old slot and the key scattered too: with the scatter 97 -> 92 us for
-// 3.0 M particles, 143 -> 126 for 4.5 M); also rebuilds the views and resets the per-case maximum speed slots and the path
-// lengths of this step.
+// 3.0 M particles, 143 -> 126 for 4.5 M); also rebuilds the views and resets the per-case maximum
+// speed slots and the path lengths of this step.
 template <class Pol>
 __global__ void __launch_bounds__(256) k_permute_fluid(Dev<Pol> d) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1216,11 +1256,12 @@ template <class Pol>
 __global__ void __launch_bounds__(64) k_umax_final(Dev<Pol> d) {
   const int c = blockIdx.x;
   if (c >= d.ncase) return;
+  const auto cap = d.cases[c].umax_cap;  // (read with the slots, not after them)
   const unsigned long long m = wave_max_u64(d.umax_slot[(size_t)(c * kSpread + (int)threadIdx.x) * kSlotStride]);
   if (threadIdx.x == 0) {
     d.umax2[c] = m;
     d.u2_last[c] = __longlong_as_double((long long)m);
-    d.umax[c] = fmin((typename Pol::R)sqrt(__longlong_as_double((long long)m)), d.cases[c].umax_cap);
+    d.umax[c] = fmin((typename Pol::R)sqrt(__longlong_as_double((long long)m)), cap);
   }
 }
 
@@ -2097,25 +2138,19 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
         });
       }
     }
-    for (int a = -1; a <= 1 && (P.sw & 2); ++a) {
-      const int jx = cx + a;
-      if (jx < 0 || jx >= cp.nx) continue;
-      const R bx = xi - cell_shift_x<Pol>(a, cp);
-      for (int b = -1; b <= 1; ++b) {
-        const int jy = cy + b;
-        if (jy < 0 || jy >= cp.ny) continue;
-        const R by = yi - cell_shift_y<Pol>(b, cp);
-        const int2 rs = d.s_range[cp.cell_off + jx * cp.ny + jy];
-        for_range<2>(rs.x, rs.y, [&](int k) {  // fluidSolidCalculate: rho_j = rho_i
-          const int j = d.s_sorted[k];
-          const R dx = d.s_vx[j] - bx, dy = d.s_vy[j] - by;
-          const R r2 = norm2(dx, dy);
-          if (!(r2 < K.rc2)) return;
-          const R w = K.w_in(r2);
-          const R du_ = ui - (R)d.su[j], dv_ = vi - (R)d.sv[j];
-          riemann_pair<R, VISCID>(dx, dy, r2, kfma(du_, dx, dv_ * dy), w, du_, dv_, rhoi, d.s_p[j], I, S);
-        });
-      }
+    if (P.sw & 2) {  // fluidSolidCalculate: rho_j = rho_i
+      struct Sol {
+        R u, v, p;
+      };
+      for_cell_solids<Pol, 4>(
+          d, cp, cx, cy, xi, yi, [&](int j) { return Sol{(R)d.su[j], (R)d.sv[j], d.s_p[j]}; },
+          [&](R dx, R dy, const Sol &q) {
+            const R r2 = norm2(dx, dy);
+            if (!(r2 < K.rc2)) return;
+            const R w = K.w_in(r2);
+            const R du_ = ui - q.u, dv_ = vi - q.v;
+            riemann_pair<R, VISCID>(dx, dy, r2, kfma(du_, dx, dv_ * dy), w, du_, dv_, rhoi, q.p, I, S);
+          });
     }
     pair_finish(S, I);
     d.f_col[i] = S.col;
