@@ -40,3 +40,33 @@ def test_fluid_force_on_solids_matches_the_oracle(gpu, oracle_mod, precision, to
     assert np.count_nonzero(want) > 0
     assert np.linalg.norm(got - want) <= tol * np.linalg.norm(want)
     assert np.array_equal(got == 0, want == 0)
+
+
+# The fluid's increments of velocity and density: P64 to the 1e-9 bar, M32 to 1e-4 (sums of float
+# terms of both signs, each to a few 1e-7, that cancel to some tenth of the largest).
+@pytest.mark.parametrize("precision,tol", [("p64", 1e-9), ("m32", 1e-4)])
+@pytest.mark.parametrize("solids_per_cell", [0.2, 2, 9, 30])
+def test_solid_terms_of_the_fluid_match_the_oracle(gpu, oracle_mod, precision, tol, solids_per_cell):
+    p = params(gravity=0.0, dt=1e-5, shift_per_step=0)
+    rc = 3.0 * p.smoothing_length
+    rng = np.random.default_rng(int(10 * solids_per_cell) + 2)
+    lo, hi = p.domain_xmin + 1e-6, p.domain_xmax - 1e-6
+    n = int(solids_per_cell * ((hi - lo) / rc) ** 2)
+    sx, sy = rng.uniform(lo, hi, n), rng.uniform(lo, hi, n)
+    keep = ~((sx > 0.7) & (sy > 0.7)) & ~((sx > 0.35) & (sx < 0.35 + 1.5 * rc))  # cells without any
+    sx, sy = sx[keep], sy[keep]
+    x, y = rng.uniform(lo, hi, 600), rng.uniform(lo, hi, 600)
+    far = ((x[:, None] - sx) ** 2 + (y[:, None] - sy) ** 2).min(1) > (0.05 * rc) ** 2
+    x, y = x[far], y[far]
+    m = len(x)
+    u, v = rng.normal(0, 3, m), rng.normal(0, 3, m)
+    c = case(p, fluid(x, y, u=u, v=v, p=rng.uniform(0, 900, m)),
+             solid(sx, sy, u=rng.normal(0, 3, len(sx)), v=rng.normal(0, 3, len(sx))))
+    sim, ora = Simulation(c, precision), oracle_mod.Oracle(c)
+    for st in ("cells", "couple", "wall", "fluid"):
+        sim.stage(st)
+        ora.stage(st)
+    a, b = sim.download()["fluid"], ora.download()["fluid"]
+    for f, f0 in (("u", u), ("v", v), ("rho", 1000.0)):
+        want = b[f] - f0
+        assert np.linalg.norm((a[f] - f0) - want) <= tol * np.linalg.norm(want), f
