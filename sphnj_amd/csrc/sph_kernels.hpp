@@ -3221,9 +3221,11 @@ __device__ __forceinline__ void grid_sync(const GridSync &g, unsigned e, int spi
 
 // d0 is the state as the sub-steps begin; d1 the same with every ping-pong pair of solid
 // buffers swapped (odd sub-steps read what even ones wrote).  The host swaps its own pointers
-// S times after the launch, as after 2 S launches.
+// S times after the launch, as after 2 S launches.  M32 is held to 128 registers, so that a CU holds
+// two blocks and the 6.3 k solids of the 288 k gate fit half the device in one round (one register
+// more halved the grid: 250 -> 296 us per step).
 template <class Pol>
-__global__ void __launch_bounds__(kSubstepBlock) k_solid_substeps(Dev<Pol> d0, Dev<Pol> d1, int S, GridSync g,
+__global__ void __launch_bounds__(kSubstepBlock, Pol::MIXED ? 4 : 2) k_solid_substeps(Dev<Pol> d0, Dev<Pol> d1, int S, GridSync g,
                                                                   int spin_limit) {
   const int n = d0.ns * kSolidLanes, stride = (int)(gridDim.x * blockDim.x);
   unsigned e = 0;
