@@ -46,7 +46,7 @@ BYTES = {
     # the double masters, L, u, v and writes the masters, u, v (133 B).  P64: the positions are
     # the views, the accumulated shift and L are double (69, 85 and 141 B).
     "shift": {"m32": 60, "p64": 89},
-    "cells": {"m32": 16 + 142, "p64": 20 + 150},   # hash + sort/permute/cell ranges
+    "cells": {"m32": 16 + 134, "p64": 20 + 142},   # hash + sort/permute/cell ranges
 }
 WALL_BYTES = {"m32": 38, "p64": 66}  # wall Shepard, per wall particle
 

@@ -1708,7 +1708,7 @@ inline bool pair_wide(int B, double q) {
 }
 // The shift stages three quarters of the pair's budget: tiles over both sub-columns of a cell
 // column stage about 3.4 candidates a lane (a dense 256-lane tile ~870), and the smaller LDS
-// lets 8 blocks of 256 share a CU.
+// leaves the count of 256-lane blocks on a CU (seven) to the registers.
 template <int BLOCK>
 struct ShiftCap {
   static constexpr int value = plan_cap(BLOCK) * 3 / 4;
