@@ -1360,17 +1360,19 @@ __device__ __forceinline__ LanePos lane_pos_view(float xi, float yi, int cx, int
 constexpr int kWindowOrder = 7;
 __device__ __forceinline__ int window_offset(int q) { return (q & 1) ? -((q + 1) >> 1) : (q >> 1); }
 
-// Visits the candidate row windows of a lane of sub-column sx: f(sc, ra, rb) for each
+// Visits the candidate row windows of a lane of sub-column sx: f(sc, ra, rb, cut) for each
 // sub-column sc that meets the lane's disc of radius R, with the sub-rows [ra, rb] that do,
 // clipped to the 3x3 cells of the lane's cell (the tile's cell column, row cy) and to the
 // tile's candidate range; sub-columns in window_offset order (PAIRED) or from left to right.
+// cut: the disc reaches sub-rows of the tile above the 3x3 cells, whose particles are none of
+// the lane's candidates however near they come.
 template <bool PAIRED, class CP, class F>
 __device__ __forceinline__ void for_windows(const TilePlan &P, const CP &cp, int sx, int sy, int cy, LanePos lp,
                                             float R, F &&f) {
   const float R2 = R * R;
   const int a_lo = max((int)floorf(lp.fx - R * cp.inv_ssx), P.sc0 - sx);
   const int a_hi = min((int)floorf(lp.fx + R * cp.inv_ssx), P.sc0 + P.nsc - 1 - sx);
-  const int rmin = max(2 * cy - 2, P.r0), rmax = min(2 * cy + 3, P.r0 + P.nr - 1);
+  const int rmin = max(2 * cy - 2, P.r0), rmax = P.r0 + P.nr - 1;
   for (int q = PAIRED ? 0 : a_lo; q < (PAIRED ? kWindowOrder : a_hi + 1); ++q) {
     const int a = PAIRED ? window_offset(q) : q;
     if (PAIRED && (a < a_lo || a > a_hi)) continue;
@@ -1378,8 +1380,8 @@ __device__ __forceinline__ void for_windows(const TilePlan &P, const CP &cp, int
     if (g >= R) continue;
     const float hr = fminf(__builtin_amdgcn_sqrtf(R2 - g * g) * cp.inv_ssy, 8.f);
     const int ra = max(sy + (int)floorf(lp.fy - hr), rmin);
-    const int rb = min(sy + (int)floorf(lp.fy + hr), rmax);
-    if (ra <= rb) f(sx + a, ra, rb);
+    const int top = min(sy + (int)floorf(lp.fy + hr), rmax), rb = min(top, 2 * cy + 3);
+    if (ra <= rb) f(sx + a, ra, rb, top > rb);
   }
 }
 
@@ -1387,7 +1389,7 @@ __device__ __forceinline__ void for_windows(const TilePlan &P, const CP &cp, int
 // (for_windows for one sub-column); false when the sub-column holds no candidate of the lane.
 template <class CP>
 __device__ __forceinline__ bool span_window(const TilePlan &P, const CP &cp, int sx, int sa, int sy, int cy,
-                                            LanePos lp, float R, int &ra, int &rb) {
+                                            LanePos lp, float R, int &ra, int &rb, bool &cut) {
   if (sa < 0 || sa >= P.nsc) return false;
   const int a = P.sc0 + sa - sx;
   const float R2 = R * R;
@@ -1396,7 +1398,9 @@ __device__ __forceinline__ bool span_window(const TilePlan &P, const CP &cp, int
   if (g >= R) return false;
   const float hr = fminf(__builtin_amdgcn_sqrtf(R2 - g * g) * cp.inv_ssy, 8.f);
   ra = max(sy + (int)floorf(lp.fy - hr), max(2 * cy - 2, P.r0));
-  rb = min(sy + (int)floorf(lp.fy + hr), min(2 * cy + 3, P.r0 + P.nr - 1));
+  const int top = min(sy + (int)floorf(lp.fy + hr), P.r0 + P.nr - 1);
+  rb = min(top, 2 * cy + 3);
+  cut = top > rb;
   return ra <= rb;
 }
 
@@ -1425,8 +1429,12 @@ __device__ __forceinline__ bool span_window(const TilePlan &P, const CP &cp, int
 // first pass would), and every pass of the step is a kShiftCached one: the paths then count
 // from the hash, which bounds the paths since the recording.
 //   A run is walked in whole groups of kRunPad + 1 (M32 4, P64 2: its four candidates' FP64 terms
-// in flight cost more registers than they hide): entries past its end lie beyond rc (its span's
-// next candidates) or far away (the padding), and add exact zeros.
+// in flight cost more registers than they hide).  The entries that the last group reads past the run
+// are far away (the padding) or particles of the span beyond rc (1 + s) at the recording -- the
+// window's others, or those that its pruning left out -- and add exact zeros.  Particles that only the
+// clip to the 3x3 cells left out can come within rc (they lie a cell's height away, which exceeds rc by
+// as little as 1/2000), so a run whose groups would reach past such a clip is recorded with the missing
+// entries before its start instead (RunRec::put).
 template <class Pol>
 constexpr int kRunPad = Pol::MIXED ? 3 : 1;
 constexpr int kShiftPlain = 0, kShiftRecord = 1, kShiftCached = 2;
@@ -1435,12 +1443,25 @@ constexpr double kShiftSkin = 0.02;
 // A lane's recorded candidate runs, in the packing of f_wc: up to 5 runs of (11-bit start,
 // 7-bit length) in three words; ok turns false at a sixth run, a run past 127 slots or a start
 // past 2047 (the lane then searches its full windows).
+template <int PAD>
 struct RunRec {
   unsigned w0 = 0u, w1 = 0u, w2 = 0u;
   int n = 0;
   bool ok = true;
-  __device__ __forceinline__ void put(int f, int len) {
-    if (n >= 5 || len > 127 || f > 2047) {
+  // The run of len entries from f on, of the window [s0, s1) of span sa.  cut: entries from s1 on may
+  // come within rc, so the walk ends with the run and whole groups start before it: there lie the
+  // window's others, what the window's pruning left out (unless the window starts with the 3x3 cells
+  // too, low: a disc of 3/2 cell heights) and the padding of the span before.
+  __device__ __forceinline__ void put(int f, int len, int sa, int s0, int s1, bool cut, bool low) {
+    static_assert((PAD & (PAD + 1)) == 0, "groups of a power of two");
+    const int more = -len & PAD;
+    f += PAD * sa;  // as a kShiftCached pass stages it
+    if (cut && f + len + more > s1 + PAD * sa) {
+      f -= more;
+      len += more;
+      ok = ok && !(low && f < s0 + PAD * sa);
+    }
+    if (n >= 5 || len > 127 || (unsigned)f > 2047u) {
       ok = false;
       return;
     }
@@ -1930,7 +1951,7 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
       // in-range mask of the run [s0, s1) of at most 32 candidates; with REC also the mask ms
       // of the candidates within rc (1 + s) (the recorded runs).  A longer run is evaluated
       // whole (direct), in its place in the window order.
-      RunRec rr;
+      RunRec<kRunPad<Pol>> rr;
       const R rl2 = cp.rl2_pair;
       auto direct = [&](int s0, int s1) {
         for_range_masked<2>(s0, s1, [&](int l, bool in) { staged_j(Cut{}, l, in); });
@@ -2016,7 +2037,8 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
         w0[q] = 0;
         const int sa = off + o;
         int ra, rb;
-        if (!span_window(P, cp, lsx, sa, sy, cy, lp, Rpw, ra, rb)) continue;
+        bool cut;
+        if (!span_window(P, cp, lsx, sa, sy, cy, lp, Rpw, ra, rb, cut)) continue;
         const int s0 = s_lb[sa][ra - P.r0], s1 = s_lb[sa][rb + 1 - P.r0];
         w0[q] = s0;
         if (s1 - s0 > 32) {  // evaluated whole below
@@ -2029,7 +2051,7 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
           mk[q] = mark(std::true_type{}, s0, s1, ms);
           if (ms != 0u) {
             const int f = __builtin_ctz(ms);
-            rr.put(s0 + kRunPad<Pol> * sa + f, 32 - __builtin_clz(ms) - f);
+            rr.put(s0 + f, 32 - __builtin_clz(ms) - f, sa, s0, s1, cut, ra == 2 * cy - 2);
           }
         } else {
           mk[q] = mark(std::false_type{}, s0, s1, ms);
@@ -2057,7 +2079,8 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
           for (int h = 0; h < 2; ++h) {
             const int sa = off + window_offset(q + h);
             int ra, rb;
-            if ((h == 1 && k == 0) || !span_window(P, cp, lsx, sa, sy, cy, lp, Rpw, ra, rb)) continue;
+            bool cut;
+            if ((h == 1 && k == 0) || !span_window(P, cp, lsx, sa, sy, cy, lp, Rpw, ra, rb, cut)) continue;
             s0[h] = s_lb[sa][ra - P.r0];
             s1[h] = s_lb[sa][rb + 1 - P.r0];
             whole = whole || s1[h] - s0[h] > 32;
@@ -2106,7 +2129,7 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
       }
     }
     if (kWallLists<Pol> && record && (P.sw & 1) && !wstaged) WallList::none(d.f_wl, i);
-    for_windows<true>(P, cp, lsx, sy, cy, lp, Rp, [&](int sc, int ra, int rb) {
+    for_windows<true>(P, cp, lsx, sy, cy, lp, Rp, [&](int sc, int ra, int rb, bool) {
       if (staged) return;
       const R bx = xi - cell_shift_x<Pol>((sc >> 1) - cx, cp);
       if constexpr (Pol::MIXED) {
@@ -2362,7 +2385,7 @@ __device__ __forceinline__ void shift_tile(const Dev<Pol> &d, const TilePlan &P,
   };
   auto staged_add = [&](int l, bool) { (void)staged_term(l); };
   // first pass of several: the runs to record (see kShiftRecord)
-  RunRec rr;
+  RunRec<kRunPad<Pol>> rr;
   rr.ok = staged;
   if (cached) {
     const unsigned x = own.wc.x, y = own.wc.y, z = own.wc.z;
@@ -2381,7 +2404,7 @@ __device__ __forceinline__ void shift_tile(const Dev<Pol> &d, const TilePlan &P,
     walk(s4, (int)(z >> 25));
   } else {
     const R rl2 = cp.rl2_rec;
-    for_windows<false>(P, cp, lsx, sy, cy, lp, Rp, [&](int sc, int ra, int rb) {
+    for_windows<false>(P, cp, lsx, sy, cy, lp, Rp, [&](int sc, int ra, int rb, bool cut) {
       if (staged) {
         const int sa = sc - P.sc0;
         const int lo = s_lb[sa][ra - P.r0], hi = s_lb[sa][rb + 1 - P.r0];
@@ -2408,7 +2431,7 @@ __device__ __forceinline__ void shift_tile(const Dev<Pol> &d, const TilePlan &P,
             if (l < hi) mk |= (staged_term(l) < rl2 ? 1u : 0u) << sh;
             if (mk != 0u) {
               const int f = __builtin_ctz(mk);
-              rr.put(lo + kRunPad<Pol> * sa + f, 32 - __builtin_clz(mk) - f);
+              rr.put(lo + f, 32 - __builtin_clz(mk) - f, sa, lo, hi, cut, ra == 2 * cy - 2);
             }
           } else {  // f follows l until one is seen
             int f = lo, la = lo;
@@ -2419,7 +2442,7 @@ __device__ __forceinline__ void shift_tile(const Dev<Pol> &d, const TilePlan &P,
               seen = seen || in;
               la = in ? q : la;
             });
-            if (seen) rr.put(f + kRunPad<Pol> * sa, la - f + 1);
+            if (seen) rr.put(f, la - f + 1, sa, lo, hi, cut, ra == 2 * cy - 2);
           }
         } else {
           for_range_4_2_1(lo, hi, staged_add);
