@@ -3376,6 +3376,7 @@ constexpr int kGatherMax = 14;
 struct GatherArgs {
   GatherField f[kGatherMax];
   int nf, n, lo;    // fields, particles, the case's first slot
+  int o0, m;        // the particles of input indices [o0, o0 + m), to dst from its start on
   const int *orig;  // slot -> global original index (null: slots are in input order)
 };
 // A thread per slot: slots in order read whole lines, and slots that are neighbours in space have
@@ -3383,7 +3384,8 @@ struct GatherArgs {
 __global__ void __launch_bounds__(256) k_gather(GatherArgs a) {
   const int i = blockIdx.x * 256 + (int)threadIdx.x;
   if (i >= a.n) return;
-  const int s = a.lo + i, o = a.orig ? a.orig[s] - a.lo : i;
+  const int s = a.lo + i, o = (a.orig ? a.orig[s] - a.lo : i) - a.o0;
+  if (o < 0 || o >= a.m) return;
   for (int k = 0; k < a.nf; ++k) {
     const GatherField f = a.f[k];
     if (f.bytes == 8)

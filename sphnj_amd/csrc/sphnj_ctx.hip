@@ -7,7 +7,6 @@
 #include <algorithm>
 #include <climits>
 #include <array>
-#include <atomic>
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -714,6 +713,7 @@ struct Engine : EngineBase {
         if ((rc = dalloc(&d.s_ref_j, 1)) || (rc = dalloc(&d.s_ref_g, 2))) return rc;
       }
     }
+    if ((rc = init_stage())) return rc;
     // hash and order the fluid and solid once, so every stage finds valid cells
     if ((rc = stage_cells(false))) return rc;
     HIPC(hipStreamSynchronize(stream));
@@ -1217,15 +1217,32 @@ struct Engine : EngineBase {
   // widening and the caller's page faults of others (a stream per thread would copy no faster and
   // costs about 3 ms to create).  All 15 fluid fields of the 3.0 M two-phase dam break: 9 ms (61 to 80
   // with a pageable copy per field and a scatter by the calling thread); of 800 particles:
-  // 70 us (280).  Staging, slices and events belong to the context and are kept.
-  static constexpr size_t kInlineBytes = (size_t)3 << 20, kPieceBytes = (size_t)1 << 20;
+  // 70 us (280).
+  //   The staging is bounded: what does not fit is gathered in rounds by input index, each by the
+  // thread that takes the round's first piece (pieces are taken and enqueued under one lock, so a
+  // round's gather follows the copies of the round before).  Its first kInlineBytes, or less where no
+  // download is larger, belong to the context from the start; up to kStageMax is taken when a download
+  // first asks for it (3.0 M particles take 9.1 ms, with 256 MiB 9.3, with room for everything at once
+  // 9.3), and without it (a device with no memory left) the rounds are smaller (16 ms).
+  static constexpr size_t kInlineBytes = (size_t)3 << 20, kPieceBytes = (size_t)1 << 20, kStageMax = (size_t)64 << 20;
   static constexpr int kCopyThreads = 8;
-  struct OutField {  // n particles of w elements of esize bytes from staging at off
-    size_t off;
-    int esize, w, n;
+  struct OutField {  // n particles of w elements of esize bytes
+    int esize, w;
     double *d;
     int32_t *i;
   };
+  struct OutJob {  // the fields of one species
+    GatherArgs a{};
+    OutField f[kGatherMax];
+    size_t bytes = 0;  // of a particle
+    size_t need() const { return a.n * bytes + kStageAlign * a.nf; }
+  };
+  struct OutChunk {  // m elements of a field from element e0 on, from staging at off
+    OutField f;
+    size_t off, e0, m;
+    int round;
+  };
+  static constexpr size_t kStageAlign = 256;
   char *stage_dev = nullptr, *stage_pin = nullptr;
   size_t stage_cap = 0, pin_cap = 0;
   hipEvent_t copy_ev[kCopyThreads] = {};
@@ -1242,38 +1259,63 @@ struct Engine : EngineBase {
       for (size_t k = 0; k < m; ++k) f.i[e0 + k] = (int32_t)q[k];
     }
   }
-  // memory of at least `need` bytes in *p, kept for later calls
-  int grow(char **p, size_t *cap, size_t need, bool pinned) {
-    if (*cap >= need) return SPHNJ_OK;
-    if (*p) HIPC(pinned ? hipHostFree(*p) : hipFree(*p));
-    *p = nullptr;
-    *cap = 0;
-    if (pinned)
-      HIPC(hipHostMalloc((void **)p, need, hipHostMallocDefault));
-    else
-      HIPC(hipMalloc((void **)p, need));
-    *cap = need;
+  // device staging of `need` bytes, kept for later calls; what there is if that cannot be had
+  void grow_stage(size_t need) {
+    if (stage_cap >= need) return;
+    void *p = nullptr;
+    if (hipMalloc(&p, need) != hipSuccess) {
+      (void)hipGetLastError();
+      return;
+    }
+    if (stage_dev) (void)hipFree(stage_dev);
+    stage_dev = (char *)p;
+    stage_cap = need;
+  }
+  // pinned memory of `need` bytes, kept for later calls; pageable memory of this call if there is none
+  char *grow_pin(size_t need, std::vector<char> &pageable) {
+    if (pin_cap < need) {
+      void *p = nullptr;
+      if (hipHostMalloc(&p, need, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        pageable.resize(need);
+        return pageable.data();
+      }
+      if (stage_pin) (void)hipHostFree(stage_pin);
+      stage_pin = (char *)p;
+      pin_cap = need;
+    }
+    return stage_pin;
+  }
+  // the staging that a context has from the start: the largest download of a case, kInlineBytes at most
+  int init_stage() {
+    size_t most = 0;
+    for (int c = 0; c < ncase; ++c) {
+      const size_t bf = 5 * 8 + 6 * sizeof(R) + 3, bs = 8 * 8 + 21 * sizeof(R), bw = 2 * 8 + 6 * sizeof(R) + 2;
+      most = std::max(most, bf * (f_off[c + 1] - f_off[c]) + bs * (s_off[c + 1] - s_off[c]) +
+                                bw * (w_off[c + 1] - w_off[c]) + 3 * kGatherMax * kStageAlign);
+    }
+    most = std::min(most, kInlineBytes);
+    HIPC(hipMalloc((void **)&stage_dev, most));
+    stage_cap = most;
     return SPHNJ_OK;
   }
 
   int download(int c, const sphnj_fluid_out *f, const sphnj_solid_out *s, const sphnj_wall_out *w) override {
-    std::vector<OutField> out;
-    std::vector<GatherArgs> jobs;
-    size_t total = 0;
-    auto add = [&](GatherArgs &J, const auto *src, int wd, double *dd, int32_t *ii) {
-      if (!src || (!dd && !ii) || J.n == 0) return;
+    std::vector<OutJob> jobs;
+    auto add = [&](OutJob &J, const auto *src, int wd, double *dd, int32_t *ii) {
+      if (!src || (!dd && !ii) || J.a.n == 0) return;
       const int es = (int)sizeof(*src);
-      J.f[J.nf++] = GatherField{reinterpret_cast<const char *>(src), reinterpret_cast<char *>(total), es * wd};
-      out.push_back(OutField{total, es, wd, J.n, dd, ii});
-      total += ((size_t)J.n * es * wd + 255) & ~(size_t)255;
+      J.f[J.a.nf] = OutField{es, wd, dd, ii};
+      J.a.f[J.a.nf++] = GatherField{reinterpret_cast<const char *>(src), nullptr, es * wd};
+      J.bytes += es * wd;
     };
     int32_t *const no_i = nullptr;
     double *const no_d = nullptr;
     if (f) {
-      GatherArgs J{};
-      J.n = f_off[c + 1] - f_off[c];
-      J.lo = f_off[c];
-      J.orig = d.f_orig;
+      OutJob J;
+      J.a.n = f_off[c + 1] - f_off[c];
+      J.a.lo = f_off[c];
+      J.a.orig = d.f_orig;
       add(J, d.fa.x, 1, f->x, no_i);
       add(J, d.fa.y, 1, f->y, no_i);
       add(J, d.fa.u, 1, f->u, no_i);
@@ -1285,12 +1327,12 @@ struct Engine : EngineBase {
       add(J, d.f_phase, 1, no_d, f->phase);
       add(J, d.f_cls, 1, no_d, f->boundary_type);
       add(J, d.f_near, 1, no_d, f->near);
-      if (J.nf) jobs.push_back(J);
+      if (J.a.nf) jobs.push_back(J);
     }
     if (s) {  // solids stay in input order
-      GatherArgs J{};
-      J.n = s_off[c + 1] - s_off[c];
-      J.lo = s_off[c];
+      OutJob J;
+      J.a.n = s_off[c + 1] - s_off[c];
+      J.a.lo = s_off[c];
       add(J, d.sx, 1, s->x, no_i);
       add(J, d.sy, 1, s->y, no_i);
       add(J, d.su, 1, s->u, no_i);
@@ -1305,13 +1347,13 @@ struct Engine : EngineBase {
       add(J, d.s_P, 4, s->stress, no_i);
       add(J, d.s_M, 4, s->max_strain, no_i);
       add(J, d.s_cp, 2, s->couple_dudt, no_i);
-      if (J.nf) jobs.push_back(J);
+      if (J.a.nf) jobs.push_back(J);
     }
     if (w) {
-      GatherArgs J{};
-      J.n = w_off[c + 1] - w_off[c];
-      J.lo = w_off[c];
-      J.orig = d.w_orig;
+      OutJob J;
+      J.a.n = w_off[c + 1] - w_off[c];
+      J.a.lo = w_off[c];
+      J.a.orig = d.w_orig;
       add(J, d.wx, 1, w->x, no_i);
       add(J, d.wy, 1, w->y, no_i);
       add(J, d.w_u, 1, w->u, no_i);
@@ -1321,59 +1363,99 @@ struct Engine : EngineBase {
       add(J, d.w_n, 2, w->normal, no_i);
       add(J, d.w_phase, 1, no_d, w->phase);
       add(J, d.w_bc, 1, no_d, w->bc);
-      if (J.nf) jobs.push_back(J);
+      if (J.a.nf) jobs.push_back(J);
     }
-    const bool inl = total <= kInlineBytes;
-    int rc;
-    if (total > 0) {
-      if ((rc = grow(&stage_dev, &stage_cap, total, false)) ||
-          (rc = grow(&stage_pin, &pin_cap, inl ? total : std::max(pin_cap, kCopyThreads * kPieceBytes), true)))
-        return rc;
-      for (GatherArgs &J : jobs) {
-        for (int k = 0; k < J.nf; ++k) J.f[k].dst = stage_dev + reinterpret_cast<size_t>(J.f[k].dst);
-        k_gather<<<nblk(J.n, 256), 256, 0, stream>>>(J);
+    size_t need = 0;
+    for (const OutJob &J : jobs) need += J.need();
+    grow_stage(std::min(need, kStageMax));
+    // the rounds: what is gathered in each, and where the fields lie
+    std::vector<std::vector<GatherArgs>> rounds(1);
+    std::vector<OutChunk> chunks;
+    size_t used = 0;
+    for (const OutJob &J : jobs) {
+      const size_t pad = kStageAlign * J.a.nf;
+      for (int o = 0; o < J.a.n;) {
+        const size_t m = used + pad < stage_cap ? std::min<size_t>(J.a.n - o, (stage_cap - used - pad) / J.bytes) : 0;
+        if (m == 0) {
+          if (used == 0) {
+            err = "download: staging too small for a particle";
+            return SPHNJ_E_HIP;
+          }
+          rounds.emplace_back();
+          used = 0;
+          continue;
+        }
+        GatherArgs a = J.a;
+        a.o0 = o;
+        a.m = (int)m;
+        for (int k = 0; k < a.nf; ++k) {
+          const OutField &q = J.f[k];
+          a.f[k].dst = stage_dev + used;
+          chunks.push_back(OutChunk{q, used, (size_t)o * q.w, m * q.w, (int)rounds.size() - 1});
+          used += (m * q.esize * q.w + kStageAlign - 1) / kStageAlign * kStageAlign;
+        }
+        rounds.back().push_back(a);
+        o += (int)m;
       }
-      LAUNCH_CHECK();
-      if (inl) HIPC(hipMemcpyAsync(stage_pin, stage_dev, total, hipMemcpyDeviceToHost, stream));
+    }
+    auto gather = [&](int r) {
+      for (const GatherArgs &a : rounds[r]) k_gather<<<nblk(a.n, 256), 256, 0, stream>>>(a);
+      return hipGetLastError();
+    };
+    const bool inl = rounds.size() == 1 && used <= kInlineBytes;
+    std::vector<char> pageable;
+    char *const pin = grow_pin(inl ? used : kCopyThreads * kPieceBytes, pageable);
+    if (!chunks.empty()) {
+      HIPC(gather(0));
+      if (inl) HIPC(hipMemcpyAsync(pin, stage_dev, used, hipMemcpyDeviceToHost, stream));
     }
     HIPC(hipStreamSynchronize(stream));
     if (inl) {
-      for (const OutField &q : out) widen(q, stage_pin + q.off, 0, (size_t)q.n * q.w);
+      for (const OutChunk &q : chunks) widen(q.f, pin + q.off, q.e0, q.m);
       return SPHNJ_OK;
     }
-    // pieces of at most kPieceBytes, by field: (field, first element, elements)
-    struct Piece {
-      int f;
-      size_t e0, m;
-    };
-    std::vector<Piece> pieces;
-    for (size_t k = 0; k < out.size(); ++k) {
-      const size_t ne = (size_t)out[k].n * out[k].w, per = kPieceBytes / out[k].esize;
-      for (size_t e = 0; e < ne; e += per) pieces.push_back(Piece{(int)k, e, std::min(per, ne - e)});
+    // pieces of at most kPieceBytes
+    std::vector<OutChunk> pieces;
+    for (const OutChunk &q : chunks) {
+      const size_t per = kPieceBytes / q.f.esize;
+      for (size_t e = 0; e < q.m; e += per)
+        pieces.push_back(OutChunk{q.f, q.off + e * q.f.esize, q.e0 + e, std::min(per, q.m - e), q.round});
     }
     const int nt = (int)std::min<size_t>(kCopyThreads, pieces.size());
     for (int t = 0; t < nt; ++t)
       if (!copy_ev[t]) HIPC(hipEventCreateWithFlags(&copy_ev[t], hipEventDisableTiming));
     int dev = 0;
     HIPC(hipGetDevice(&dev));
-    std::atomic<size_t> next{0};
-    std::atomic<int> bad{hipSuccess};
     std::mutex enqueue;
+    size_t next = 0;                // the next piece, the round gathered last and the first error:
+    int round = 0;                  // held under the lock
+    hipError_t bad = hipSuccess;
     auto work = [&](int t) {
-      hipError_t e = hipSetDevice(dev);
-      char *const slice = stage_pin + t * kPieceBytes;
-      for (size_t k; e == hipSuccess && (k = next.fetch_add(1)) < pieces.size();) {
-        const Piece &q = pieces[k];
-        const OutField &o = out[q.f];
+      const hipError_t e0 = hipSetDevice(dev);
+      char *const slice = pin + t * kPieceBytes;
+      for (;;) {
+        const OutChunk *q;
         {
-          std::lock_guard<std::mutex> lock(enqueue);  // the event follows its own copy
-          e = hipMemcpyAsync(slice, stage_dev + o.off + q.e0 * o.esize, q.m * o.esize, hipMemcpyDeviceToHost, stream);
-          if (e == hipSuccess) e = hipEventRecord(copy_ev[t], stream);
+          // a piece is taken and its copy enqueued as one, so that the stream holds the pieces in order,
+          // each round after its gather and each event after its own copy
+          std::lock_guard<std::mutex> lock(enqueue);
+          if (bad == hipSuccess) bad = e0;
+          if (bad != hipSuccess || next == pieces.size()) return;
+          q = &pieces[next++];
+          if (q->round != round) bad = gather(round = q->round);
+          if (bad == hipSuccess)
+            bad = hipMemcpyAsync(slice, stage_dev + q->off, q->m * q->f.esize, hipMemcpyDeviceToHost, stream);
+          if (bad == hipSuccess) bad = hipEventRecord(copy_ev[t], stream);
+          if (bad != hipSuccess) return;
         }
-        if (e == hipSuccess) e = hipEventSynchronize(copy_ev[t]);
-        if (e == hipSuccess) widen(o, slice, q.e0, q.m);
+        const hipError_t e = hipEventSynchronize(copy_ev[t]);
+        if (e != hipSuccess) {
+          std::lock_guard<std::mutex> lock(enqueue);
+          bad = e;
+          return;
+        }
+        widen(q->f, slice, q->e0, q->m);
       }
-      if (e != hipSuccess) bad = (int)e;
     };
     std::vector<std::thread> th;
     th.reserve(nt);
@@ -1384,7 +1466,8 @@ struct Engine : EngineBase {
     work(0);
     for (std::thread &t : th) t.join();
     if (bad != hipSuccess) {
-      err = std::string("download: ") + hipGetErrorString((hipError_t)bad.load());
+      (void)hipStreamSynchronize(stream);  // no copy into the slices is left in flight
+      err = std::string("download: ") + hipGetErrorString(bad);
       return SPHNJ_E_HIP;
     }
     return SPHNJ_OK;
