@@ -171,7 +171,8 @@ struct alignas(16) Dev {
   // per cell column (case offset swp_off), ny + 1 entries: first wall slot of cell row k or
   // later, the column's end last (walls are sorted by cell once)
   int *w_lb;
-  // P64: per slot, the walls within reach when the runs were recorded (WallList; quads nf apart)
+  // P64 with walls: per slot, the walls within reach when the runs were recorded (WallList; quads nf
+  // apart; null where there was no memory for them)
   uint4 *f_wl;
 };
 

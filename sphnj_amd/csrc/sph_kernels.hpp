@@ -823,7 +823,8 @@ struct alignas(16) TilePlan {  // (read by scalar loads)
   int sx, cx, gcol;      // even sub-column and cell column of the tile; global cell column
   int sc0, nsc, r0, nr;  // candidate sub-columns and sub-rows
   int cy_ref;            // cell row of the M32 shift frame
-  int sw;                // wall (bit 0) / solid (bit 1) particles lie in the tile's 3x3 cells
+  int sw;                // wall (bit 0) / solid (bit 1) particles lie in the tile's 3x3 cells; bit 2: with
+                         // walls, and their lists have memory (f_wl)
   int total;             // candidate particles (sum of the span lengths)
   int lo[kTileCols], len[kTileCols], row[kTileCols];  // slot span; f_lb index of (sc0 + a, r0)
   int gsz, gmul;         // staging: threads per span B / nsc; ceil(2^20 / gsz) (t / gsz = t gmul >> 20)
@@ -1186,7 +1187,7 @@ __global__ void __launch_bounds__(256) k_tile_plan(Dev<Pol> d, int G, const int 
     P.r0 = r0;
     P.nr = nr;
     P.cy_ref = (sy0 + sy1) >> 2;
-    P.sw = (nw > 0 ? 1 : 0) | (ns > 0 ? 2 : 0);
+    P.sw = (nw > 0 ? 1 : 0) | (ns > 0 ? 2 : 0) | (nw > 0 && d.f_wl != nullptr ? 4 : 0);
     P.total = total;
     P.gsz = B / nsc;
     P.gmul = ((1 << 20) + P.gsz - 1) / P.gsz;
@@ -2113,7 +2114,7 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
         // evaluated whole they made the walls' waves the slowest of a launch)
         const int lr0 = max(cy - 1, 0) - W.wcr0, lr1 = min(cy + 1, cp.ny - 1) - W.wcr0;
         // (a recording also lists the walls within rc (1 + s), in this order, for the shift passes)
-        WallList wl(W.n);
+        WallList wl((P.sw & 4) ? W.n : 256);
 #pragma unroll 1
         for (int a = 0; a < 3; ++a) {
           const int s0 = s_wlb[a][lr0], s1 = s_wlb[a][lr1 + 1];
@@ -2125,10 +2126,10 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
             eval2(m, b, 0u, 0, s1 - s0 > 32);
           }
         }
-        if (kWallLists<Pol> && record) wl.close(d.f_wl, d.nf, i, W.n);
+        if (kWallLists<Pol> && record && (P.sw & 4)) wl.close(d.f_wl, d.nf, i, W.n);
       }
     }
-    if (kWallLists<Pol> && record && (P.sw & 1) && !wstaged) WallList::none(d.f_wl, i);
+    if (kWallLists<Pol> && record && (P.sw & 4) && !wstaged) WallList::none(d.f_wl, i);
     for_windows<true>(P, cp, lsx, sy, cy, lp, Rp, [&](int sc, int ra, int rb, bool) {
       if (staged) return;
       const R bx = xi - cell_shift_x<Pol>((sc >> 1) - cx, cp);
@@ -2292,7 +2293,7 @@ __device__ __forceinline__ ShiftOwn<Pol> shift_own(const Dev<Pol> &d, const Tile
       if constexpr (MODE == kShiftCached) {
         o.wc = *reinterpret_cast<const uint3 *>(d.f_wc + i);
         if (lastp) o.cum_hash = __uint_as_float(d.f_wc[i].w);
-        if (kWallLists<Pol> && (P.sw & 1)) o.wl = d.f_wl[i];
+        if (kWallLists<Pol> && (P.sw & 4)) o.wl = d.f_wl[i];
       }
     }
   }
@@ -2459,7 +2460,7 @@ __device__ __forceinline__ void shift_tile(const Dev<Pol> &d, const TilePlan &P,
   }
   if constexpr (MODE == kShiftRecord) {
     d.f_wc[i] = rr.entry(cum0);
-    if (kWallLists<Pol> && (P.sw & 1)) WallList::none(d.f_wl, i);
+    if (kWallLists<Pol> && (P.sw & 4)) WallList::none(d.f_wl, i);
   }
   // walls of the 3x3 cells (cell column by cell column, rows in order), then solids
   if (kWallLists<Pol> && wstaged && cached && (own.wl.x & 0xffu)) {  // those the recording listed, four to a word

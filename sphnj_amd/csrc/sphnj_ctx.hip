@@ -464,7 +464,6 @@ struct Engine : EngineBase {
         (rc = dalloc(&cnt_toff, (size_t)nblk(4 * nc, kScanTile) + 1)) ||
         (rc = dalloc(&d.f_col, nf)) || (rc = dalloc(&d.f_near, nf)) || (rc = dalloc(&d.f_L, 4 * (size_t)nf)) ||
         (rc = dalloc(&d.f_sacc, 2 * (size_t)nf)) || (rc = dalloc(&d.f_wc, nf)) ||
-        (rc = dalloc(&d.f_wl, kWallLists<Pol> ? (size_t)kWallListQuads * nf : 0)) ||
         (rc = dalloc(&d.tile_d0, (size_t)max_tiles(64))) || (rc = dalloc(&d.f_far, (size_t)G)) ||
         (rc = dalloc(&d.f_srange, 4 * (size_t)nc)) || (rc = dalloc(&d.umax2, ncase)) || (rc = dalloc(&d.umax, ncase)) ||
         (rc = dalloc(&d.umax_slot, (size_t)ncase * kSpread * kSlotStride)) || (rc = dalloc(&d.status, 1)) ||
@@ -714,6 +713,17 @@ struct Engine : EngineBase {
       }
     }
     if ((rc = init_stage())) return rc;
+    // the wall lists only save time: where the device has no memory left for them, the shift passes walk
+    // their walls whole
+    if (kWallLists<Pol> && nw > 0 && nf > 0) {
+      void *q = nullptr;
+      if (hipMalloc(&q, (size_t)kWallListQuads * nf * sizeof(uint4)) == hipSuccess) {
+        allocs.push_back(q);
+        d.f_wl = (uint4 *)q;
+      } else {
+        (void)hipGetLastError();
+      }
+    }
     // hash and order the fluid and solid once, so every stage finds valid cells
     if ((rc = stage_cells(false))) return rc;
     HIPC(hipStreamSynchronize(stream));

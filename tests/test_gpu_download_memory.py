@@ -49,3 +49,19 @@ def test_download_takes_bounded_device_memory(gpu, precision):
             assert np.array_equal(got["solid"][k], s[k]), k
         for k in ("x", "y", "bc"):
             assert np.array_equal(got["wall"][k], w[k]), k
+
+
+def test_wall_lists_take_no_memory_without_walls(gpu):
+    """The P64 shift passes' wall lists (48 bytes a fluid particle) belong to contexts with walls only:
+    a context without takes that much less than the same with one wall (4 MiB of slack)."""
+    n = 1024
+    x, y = lattice(n, n, 8.5e-4, 0.05, 0.05)
+    p = params(particle_diameter=8.5e-4, smoothing_length=1.105e-3)
+    taken = []
+    Simulation(case(p, fluid(x, y), None, wall([0.02], [0.02])), "p64").close()  # (loads the kernels)
+    for w in (None, wall([0.02], [0.02])):
+        before = free_memory()
+        sim = Simulation(case(p, fluid(x, y), None, w), "p64")
+        taken.append(before - free_memory())
+        sim.close()
+    assert taken[1] - taken[0] >= 48 * n * n - (4 << 20)
