@@ -6,6 +6,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <stddef.h>
 #include <stdint.h>
 
 #include <type_traits>
@@ -89,7 +90,7 @@ struct FluidBuf {
 
 // The order and the alignment count: the compiler reads the pointers in wide scalar loads where
 // they lie on multiples of them, and eight bytes more or less ahead of the others cost the M32 shift
-// and pair kernels 1 to 4 %.
+// and pair kernels 1 to 4 % (asserted below).
 template <class Pol>
 struct alignas(16) Dev {
   using R = typename Pol::R;
@@ -175,6 +176,11 @@ struct alignas(16) Dev {
   // apart; null where there was no memory for them)
   uint4 *f_wl;
 };
+template <class Pol>
+constexpr bool kDevAligned = offsetof(Dev<Pol>, fa) % 16 == 0 && offsetof(Dev<Pol>, fb) % 16 == 0 &&
+                             offsetof(Dev<Pol>, f_phase) % 16 == 0 && offsetof(Dev<Pol>, f_srange) % 16 == 0 &&
+                             offsetof(Dev<Pol>, sx) % 16 == 0;
+static_assert(kDevAligned<M32> && kDevAligned<P64>, "a new field goes last, or in pairs");
 
 // ---- helpers ----------------------------------------------------------------------------
 
