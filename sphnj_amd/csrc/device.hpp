@@ -245,7 +245,7 @@ __device__ __forceinline__ int axis_sub(double x, double x0, double inv, int n, 
 // fused multiply-add from the exact product, 2^f = 1 + f q(f) and n goes into the exponent.  q
 // (degree 10) interpolates (2^f - 1)/f at the Chebyshev nodes of the interval; with the
 // coefficients rounded to double 2^f is off by at most 2.0e-17 before the rounding of its own
-// arithmetic.  15 instructions, 14 of them FP64 (the library's exp takes about 40 with its range
+// arithmetic.  16 instructions, 14 of them FP64 (the library's exp takes about 40 with its range
 // handling).  n below -1000 gives 2^-1000 instead of leaving the exponent's range; an r2 far past
 // the cut-off (padding) gives a number that the caller's cut-off test discards.
 // FP32: v_exp_f32 computes 2^x.

@@ -1640,15 +1640,17 @@ struct PairLane {
 //   du = q / r,  (u_i - v*).dx = rho_j q / (rho_i + rho_j) - (p_i - p_j) r / ((rho_i + rho_j) c).
 // w = w'(r^2), 0 outside the cut-off.  r^2 is kept off 0 for the root only: at r = 0 every term is 0
 // through dx, dy and q; max(du, 0) takes the place of the test for an approaching pair.
-// Every multiply-add is written out and contraction is off: what a lane sums must not depend on
-// how the compiler happens to fuse an instance of the kernel (block sizes, staged or global
-// candidates), and does not.
-// M32 keeps the roundings of the separate density weights and lane factors: the classes of particles
-// at the interface hang on thresholds that a last bit can cross.  P64 forms p* from d = p_j - p_i and
+// Every multiply-add is written out and contraction is off, so that what a lane sums does not depend on
+// how the compiler happens to fuse an instance of the kernel.  In P64 every candidate's term is rounded
+// alike, whatever the block size and wherever the candidates are read.  M32 keeps, place by place, the
+// roundings that its sums have had since they were fused by the compiler (the classes of particles at
+// the interface hang on thresholds that a last bit can cross): the separate density weights and lane
+// factors, the other order of products in a loop's last candidate (swap, in eval2) and in walls that
+// are not staged (PI_FUSED).  Which candidate comes last, and what is staged, hang on the tile, so M32's
+// last bits do too.  P64 forms p* from d = p_j - p_i and
 // leaves the factors of particle i to the sums (pair_finish): fewer FP64 instructions, 922 -> 874 us
 // a launch on the 3.0 M two-phase dam break.
-// (PI_FUSED: of M32's two products in p*, p_i's is the fused one; the walls of a tile that does not
-// stage them.)
+// (PI_FUSED: of M32's two products in p*, p_i's is the fused one.)
 template <class R, bool VISCID, bool PI_FUSED = false>
 __device__ __forceinline__ void riemann_pair(R dx, R dy, R r2, R q, R w, R du_, R dv_, R rhoj, R pj,
                                              const PairLane<R> &I, PairSums<R> &A) {
@@ -1724,6 +1726,9 @@ struct PairCap {
 // over BLOCK / (2 q) sub-rows of two sub-columns, q the particles of a sub-cell, and stages six
 // sub-columns over those rows and up to 6 more, 3 BLOCK + 36 q candidates, here with 5% to spare.
 // At h/d = 1.3 (q = 4.0) that is 959 of 992 at 256 slots; past q = 4.9 the whole budget is taken.
+// Where particles crowd below that spacing d, tiles past the smaller budget read global memory; that is
+// still faster than one staged block a CU was (316 to 645 k particles: a tenth of the width at 0.8 d
+// 686 -> 371 us a launch, half at 0.7 d 1070 -> 570, all at 0.7 d 1350 -> 701).
 inline bool pair_wide(int B, double q) {
   const int cap = B < 256 ? plan_cap(B) * 5 / 8 : plan_cap(B) * 31 / 64;
   return 1.05 * (3.0 * B + 36.0 * q) > cap;
@@ -1996,8 +2001,8 @@ __global__ void __launch_bounds__(BLOCK, (Pol::MIXED ? 4 : WIDE ? 1 : 3))
         R2 p, v, r;
         int fl;
       };
-      // M32 forms r^2 and q of the last candidate with the products in the other order (swap), as
-      // the fused loop has always rounded them; not with no_swap (the lane itself, which is left
+      // M32 forms r^2 and q of the last candidate with the products in the other order (swap, see
+      // riemann_pair); not with no_swap (the lane itself, which is left
       // out, came last)
       auto eval2 = [&](unsigned ma, int sa0, unsigned mb, int sb0, bool no_swap) {
         unsigned long long m = (unsigned long long)ma | ((unsigned long long)mb << 32);
@@ -2586,8 +2591,9 @@ __device__ __forceinline__ void shift_tile(const Dev<Pol> &d, const TilePlan &P,
 // correctionCalculate (src/fluid.cu:316-367) + correctionUpdate / shiftDisplacementCalculate
 // (src/fluid.cu:369-427), one tile per block: stage the tile, then shift_tile.  MODE is
 // kShiftPlain, kShiftRecord or kShiftCached (the step's one pass, its first of several, a
-// later one).  Held to 7 waves per SIMD: vector issue bounds the M32 passes (0.95 instructions a
-// CU-cycle on the 3.0 M dam break, 92 us a pass), and an eighth wave costs spills (95 us).  Without
+// later one).  Held to 7 waves per SIMD: vector issue bounds the M32 passes (0.88 instructions a
+// CU-cycle on the 3.0 M dam break's lattice, 79 us a pass), and an eighth wave costs spills (the same
+// case with its positions disturbed 92 -> 95 us a pass, 187 k particles 18.3 -> 20.1).  Without
 // the candidates' paths in the staging and with whole groups in the runs a pass of the 187 k
 // two-phase case takes 18.3 us instead of 19.2, of the 5 k dam break 10.8 instead of 11.3, of the
 // 3.0 M case what it took (its runs' 88 slots per wave, for 45 neighbours a lane, are the rest).
@@ -3247,7 +3253,7 @@ __device__ __forceinline__ void grid_sync(const GridSync &g, unsigned e, int spi
 // buffers swapped (odd sub-steps read what even ones wrote).  The host swaps its own pointers
 // S times after the launch, as after 2 S launches.  M32 is held to 128 registers, so that a CU holds
 // two blocks and the 6.3 k solids of the 288 k gate fit half the device in one round (one register
-// more halved the grid: 250 -> 296 us per step).
+// more halved the grid: the solid stage of a step 250 -> 296 us; 243 now).
 template <class Pol>
 __global__ void __launch_bounds__(kSubstepBlock, Pol::MIXED ? 4 : 2) k_solid_substeps(Dev<Pol> d0, Dev<Pol> d1, int S, GridSync g,
                                                                   int spin_limit) {
